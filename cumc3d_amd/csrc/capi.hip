@@ -452,7 +452,7 @@ int cumc3d_init(const cumc3d_desc *desc, cumc3d_ctx **out) {
     const cumc3d_grid_metrics *gm = d.metrics;
     const double *Dm[3] = {gm ? gm->dx : nullptr, gm ? gm->dy : nullptr, gm ? gm->dz : nullptr};
     const double *Cm[3] = {gm ? gm->x : nullptr, gm ? gm->y : nullptr, gm ? gm->z : nullptr};
-    std::vector<double> hm;
+    std::vector<double> hm, hw;   // metrics, reconstruction weights
     long off[3][7];
     std::vector<double> widths[3], centres[3];
     for (int a = 0; a < 3; ++a) {
@@ -468,11 +468,11 @@ int cumc3d_init(const cumc3d_desc *desc, cumc3d_ctx **out) {
         off[a][0] = (long)hm.size(); hm.insert(hm.end(), f.begin(), f.end());
         off[a][1] = (long)hm.size(); hm.insert(hm.end(), dd.begin(), dd.end());
         off[a][2] = (long)hm.size(); hm.insert(hm.end(), cc.begin(), cc.end());
-        off[a][3] = (long)hm.size(); hm.insert(hm.end(), w.begin(), w.end());
+        off[a][3] = (long)hw.size(); hw.insert(hw.end(), w.begin(), w.end());
         // the selector's three schemes: TVD-MC, PPM, WENO-Z
         for (int sch = 0; sch < 3; ++sch) {
             weights(sch == 0 ? 2 : (sch == 1 ? 3 : 4), dd, n, w);
-            off[a][4 + sch] = (long)hm.size(); hm.insert(hm.end(), w.begin(), w.end());
+            off[a][4 + sch] = (long)hw.size(); hw.insert(hw.end(), w.begin(), w.end());
         }
     }
     // spherical metrics (getgrid.f90:68-98) and the per-index factors the
@@ -566,12 +566,23 @@ int cumc3d_init(const cumc3d_desc *desc, cumc3d_ctx **out) {
         cleanup();
         return fail(CUMC3D_EHIP, "metric upload");
     }
+    x->fp32 = d.precision == CUMC3D_FP32;
+    const size_t wsz = x->fp32 ? sizeof(float) : sizeof(double);
+    std::vector<float> hw32;
+    if (x->fp32) hw32.assign(hw.begin(), hw.end());
+    if (hipMalloc(&x->wtab, hw.size() * wsz) != hipSuccess) { cleanup(); return fail(CUMC3D_ENOMEM, "weights"); }
+    if (hipMemcpy(x->wtab, x->fp32 ? (const void *)hw32.data() : hw.data(), hw.size() * wsz, hipMemcpyHostToDevice) !=
+        hipSuccess) {
+        cleanup();
+        return fail(CUMC3D_EHIP, "weight upload");
+    }
     for (int a = 0; a < 3; ++a) {
         x->ax[a].xF = x->met + off[a][0];
         x->ax[a].d = x->met + off[a][1];
         x->ax[a].c = x->met + off[a][2];
-        x->ax[a].w = x->met + off[a][3];
-        for (int sch = 0; sch < 3; ++sch) x->ax[a].wsel[sch] = x->met + off[a][4 + sch];
+        const auto table = [&](int i) { return (const char *)x->wtab + off[a][i] * wsz; };
+        x->ax[a].w = table(3);
+        for (int sch = 0; sch < 3; ++sch) x->ax[a].wsel[sch] = table(4 + sch);
     }
     if (soff >= 0) {
         const double *b = x->met + soff;
@@ -581,8 +592,6 @@ int cumc3d_init(const cumc3d_desc *desc, cumc3d_ctx **out) {
     }
     // per-cell fields: the working-type block, then the double block, each
     // field G entries, fields 256-byte aligned
-    x->fp32 = d.precision == CUMC3D_FP32;
-    const size_t wsz = x->fp32 ? sizeof(float) : sizeof(double);
     const size_t wfield = (x->G * wsz + 255) / 256 * 256, dfield = (x->G * sizeof(double) + 255) / 256 * 256;
     const int nw = 5 + 2 + 3 + 21 + 3 + 3, nd = 6 + 8 + (x->fp32 ? 5 : 0) + 3;
     size_t bytes = nw * wfield + nd * dfield;
@@ -988,6 +997,7 @@ int cumc3d_finalize(cumc3d_ctx *x) {
     for (auto &e : x->ev) hipEventDestroy(e);
     if (x->pool) hipFree(x->pool);
     if (x->met) hipFree(x->met);
+    if (x->wtab) hipFree(x->wtab);
     if (x->S) hipFree(x->S);
     if (x->stale) hipFree(x->stale);
     if (x->grav) hipFree(x->grav);

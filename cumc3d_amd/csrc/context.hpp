@@ -22,7 +22,8 @@ struct cumc3d_ctx {
     hipStream_t stream = nullptr;
     void *pool = nullptr;         // all per-cell fields
     bool fp32 = false;            // CUMC3D_FP32: working fields are float
-    double *met = nullptr;        // grid metrics and weights
+    double *met = nullptr;        // grid metrics
+    void *wtab = nullptr;         // reconstruction weights in the working type
     cumc3d::DevScalars *S = nullptr;
     // working-type fields (double, or float in the FP32 split)
     void *P[5], *eps, *cs, *Bc[3], *F[3][7], *E[3], *Ec[3];
@@ -313,14 +314,14 @@ static void launch_sweep_rs(cumc3d_ctx *x, const ArgsT<W> &a, int D, hipStream_t
             hipLaunchKernelGGL((k_carry<W, R, 0>), dim3(1), dim3(64), 0, st, a);
     } else if (D == 1) {
         int ns = nseg_for(x, x->nx, x->nz, x->ny);
-        unsigned grid = nblk((long)x->nx * x->nz * ns);
-        hipLaunchKernelGGL((k_flux_yz<W, R, S, 1>), dim3(grid), dim3(256), 0, st, a, ns);
+        const dim3 grid(nblk((long)x->nx * x->nz), ns);
+        hipLaunchKernelGGL((k_flux_yz<W, R, S, 1>), grid, dim3(256), 0, st, a, ns);
         if (S == 3 && a.bn_mode == 2)
             hipLaunchKernelGGL((k_carry<W, R, 1>), dim3(1), dim3(64), 0, st, a);
     } else {
         int ns = nseg_for(x, x->nx, x->ny, x->nz);
-        unsigned grid = nblk((long)x->nx * x->ny * ns);
-        hipLaunchKernelGGL((k_flux_yz<W, R, S, 2>), dim3(grid), dim3(256), 0, st, a, ns);
+        const dim3 grid(nblk((long)x->nx * x->ny), ns);
+        hipLaunchKernelGGL((k_flux_yz<W, R, S, 2>), grid, dim3(256), 0, st, a, ns);
         if (S == 3 && a.bn_mode == 2)
             hipLaunchKernelGGL((k_carry<W, R, 2>), dim3(1), dim3(64), 0, st, a);
     }

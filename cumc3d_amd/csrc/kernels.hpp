@@ -44,8 +44,10 @@ struct Axis {
     const double *xF;   // face coordinate, index j+3 (j=-3..n+3)
     const double *d;    // width, index j+3
     const double *c;    // centre, index j+3
-    const double *w;    // reconstruction weights of the configured scheme, (j+3)*NW
-    const double *wsel[3];   // TVD-MC, PPM and WENO-Z weights for the learned selector
+    // reconstruction weights in the working type, (j+3)*NW: the configured
+    // scheme's, and TVD-MC, PPM and WENO-Z for the learned selector
+    const void *w;
+    const void *wsel[3];
 };
 
 // Reconstruction ids: 0 minmod, 1 van Leer, 2 MC, 3 PPM, 4 WENO-Z, and
@@ -175,10 +177,23 @@ __device__ __forceinline__ void load_stencil(const ArgsT<T> &a, long c, long st,
     }
 }
 
-template <class T> __device__ __forceinline__ void load_w(const double *w, T out[NW], int n) {
+// Weights of cell i along an axis (table of `NW` per cell in type W).  In the
+// y and z sweeps every lane of a block is at the same i, so the weights are
+// read through the constant address space: scalar loads into scalar
+// registers, which the vector instructions take as operands.
+template <class T, class W, bool UNI> __device__ __forceinline__ void load_w(const void *table, int i, T out[NW], int n) {
+    const W *w = (const W *)table + (long)(i + 3) * NW;
+    if constexpr (UNI) {
+        typedef const __attribute__((address_space(4))) W *scalar_ptr;
+        const scalar_ptr sw = (scalar_ptr)(unsigned long long)w;
 #pragma unroll
-    for (int i = 0; i < NW; ++i)
-        if (i < n) out[i] = (T)w[i];
+        for (int q = 0; q < NW; ++q)
+            if (q < n) out[q] = (T)sw[q];
+    } else {
+#pragma unroll
+        for (int q = 0; q < NW; ++q)
+            if (q < n) out[q] = (T)w[q];
+    }
 }
 
 template <int R> constexpr int nweights() { return R <= 2 ? 2 : (R == 3 ? 14 : 10); }
@@ -209,8 +224,9 @@ __device__ __forceinline__ void slide_stencil(const ArgsT<T> &a, long c, long st
     }
 }
 
-// Both faces of cell c (index i along D) from its loaded stencil.
-template <class T, int R, int D>
+// Both faces of cell c (index i along D) from its loaded stencil; UNI: the
+// lanes of a wave share i.
+template <class T, int R, int D, bool UNI>
 __device__ __forceinline__ void recon_stencil(const ArgsT<T> &a, long c, int i, const T s[7][5], Face<T> &fm,
                                               Face<T> &fp) {
     if constexpr (R == RSEL) {
@@ -221,13 +237,13 @@ __device__ __forceinline__ void recon_stencil(const ArgsT<T> &a, long c, int i, 
         const int cls = b2 ? 2 : (b1 ? 1 : 0);
         T w[NW];
         if (cls == 0) {
-            load_w<T>(a.ax[D].wsel[0] + (long)(i + 3) * NW, w, 2);
+            load_w<T, T, UNI>(a.ax[D].wsel[0], i, w, 2);
             recon_cell<T, 2>(w, s, (T)a.g1, fm, fp);
         } else if (cls == 1) {
-            load_w<T>(a.ax[D].wsel[1] + (long)(i + 3) * NW, w, 14);
+            load_w<T, T, UNI>(a.ax[D].wsel[1], i, w, 14);
             recon_cell<T, 3>(w, s, (T)a.g1, fm, fp);
         } else {
-            load_w<T>(a.ax[D].wsel[2] + (long)(i + 3) * NW, w, 10);
+            load_w<T, T, UNI>(a.ax[D].wsel[2], i, w, 10);
             recon_cell<T, 4>(w, s, (T)a.g1, fm, fp);
         }
         // positivity fallback (the selector's own, no reference counterpart):
@@ -238,7 +254,7 @@ __device__ __forceinline__ void recon_stencil(const ArgsT<T> &a, long c, int i, 
             const bool ok = fm.rho > T(0) && fp.rho > T(0) && fm.p > T(0) && fp.p > T(0);
             if (__ballot(!ok)) {
                 Face<T> gm, gp;
-                load_w<T>(a.ax[D].wsel[0] + (long)(i + 3) * NW, w, 2);
+                load_w<T, T, UNI>(a.ax[D].wsel[0], i, w, 2);
                 recon_cell<T, 2>(w, s, (T)a.g1, gm, gp);
                 if (!ok) {
                     fm = gm;
@@ -248,17 +264,17 @@ __device__ __forceinline__ void recon_stencil(const ArgsT<T> &a, long c, int i, 
         }
     } else {
         T w[NW];
-        load_w<T>(a.ax[D].w + (long)(i + 3) * NW, w, nweights<R>());
+        load_w<T, T, UNI>(a.ax[D].w, i, w, nweights<R>());
         recon_cell<T, R>(w, s, (T)a.g1, fm, fp);
     }
 }
 
-template <class T, int R, int D>
+template <class T, int R, int D, bool UNI>
 __device__ __forceinline__ void recon_at(const ArgsT<T> &a, int j, int k, int l, long st, Face<T> &fm, Face<T> &fp) {
     const long c = cidx(a, j, k, l);
     T s[7][5];
     load_stencil<T, stencil_r<R>(), D>(a, c, st, s);
-    recon_stencil<T, R, D>(a, c, (D == 0) ? j : (D == 1 ? k : l), s, fm, fp);
+    recon_stencil<T, R, D, UNI>(a, c, (D == 0) ? j : (D == 1 ? k : l), s, fm, fp);
 }
 
 template <int D, class A> __device__ __forceinline__ long stride(const A &a) {
@@ -385,7 +401,7 @@ void k_flux_x(ArgsT<T> a) {
         l = 1 + (int)(r / a.ny);
     }
     Face<T> fm, fp;
-    if (live) recon_at<T, R, 0>(a, j, k, l, 1, fm, fp);
+    if (live) recon_at<T, R, 0, false>(a, j, k, l, 1, fm, fp);
     Face<T> nm;
     nm.rho = __shfl_down(fm.rho, 1, 64);
     nm.v[0] = __shfl_down(fm.v[0], 1, 64);
@@ -416,26 +432,50 @@ void k_flux_x(ArgsT<T> a) {
     }
 }
 
-// y and z sweeps.  Threads run along x (coalesced); each thread marches along
-// the sweep axis over a segment of interfaces [i0,i1), reconstructing cells
-// i0..i1 once and keeping the previous cell's right face in registers.
+// Where a marching thread keeps the right face of the cell behind it: LDS (its
+// own column of the block's array) or registers.  The memory clobber stops the
+// compiler from carrying the slot in registers across the loop.
+template <class T> __device__ __forceinline__ void keep_face(T kept[9][256], const Face<T> &f) {
+    const int t = threadIdx.x;
+    kept[0][t] = f.rho; kept[1][t] = f.v[0]; kept[2][t] = f.v[1]; kept[3][t] = f.v[2]; kept[4][t] = f.p;
+    kept[5][t] = f.bt1; kept[6][t] = f.bt2; kept[7][t] = f.eps; kept[8][t] = f.cs;
+    __asm__ volatile("" ::: "memory");
+}
+template <class T> __device__ __forceinline__ Face<T> kept_face(const T kept[9][256]) {
+    const int t = threadIdx.x;
+    return {kept[0][t], {kept[1][t], kept[2][t], kept[3][t]}, kept[4][t], kept[5][t], kept[6][t], kept[7][t], kept[8][t]};
+}
+
+// y and z sweeps.  The cells of a plane across the sweep axis are laid end to
+// end over the threads (x fastest, coalesced) and blockIdx.y is a segment
+// [i0,i1) of interfaces along the axis: each thread marches its column over
+// the segment, reconstructing cells i0..i1 once and keeping the previous
+// cell's right face.
+// What bounds it: VALU issue, given waves to issue from.  With the kept face
+// in registers the FP64 march needed 168 to 256 VGPRs and up to 78 AGPRs (one
+// or two waves per SIMD); in LDS it needs at most 186 (three waves but for
+// HLL + WENO-Z), and the selector's 123 instead of 125 with fewer copies.
+// Measured at 256^3, y / z sweep: FP64 HLLD + WENO-Z 2.05 / 1.95 -> 1.64 /
+// 1.65 ms, FP32 selector 0.426 / 0.430 -> 0.405 / 0.409 ms.  The FP32 fixed
+// schemes keep it in registers: from LDS, TVD-MC took 0.360 against 0.353 ms
+// and PPM 0.495 against 0.474 ms.
 template <class T, int R, int S, int D>
 __global__ __launch_bounds__(256) void k_flux_yz(ArgsT<T> a, int nseg) {
     if (!a.S->active) return;
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
     const int na = (D == 1) ? a.nz : a.ny;    // the other transverse axis
     const int nd = (D == 1) ? a.ny : a.nz;    // sweep axis
-    const long total = (long)a.nx * na * nseg;
     unsigned long long key = 0;
-    if (t < total) {
-        int j = 1 + (int)(t % a.nx);
-        long rest = t / a.nx;
-        int o2 = 1 + (int)(rest % na);
-        int s = (int)(rest / na);
-        int i0 = (int)(((long)s * (nd + 1)) / nseg);
-        int i1 = (int)(((long)(s + 1) * (nd + 1)) / nseg);
+    constexpr bool lds = sizeof(T) == 8 || R == RSEL;
+    __shared__ T kept[lds ? 9 : 1][256];
+    if (t < (unsigned)a.nx * (unsigned)na) {
+        const int o2 = 1 + (int)(t / (unsigned)a.nx);
+        const int j = 1 + (int)(t - (unsigned)(o2 - 1) * (unsigned)a.nx);
+        const int s = blockIdx.y;
+        const int i0 = (int)(((long)s * (nd + 1)) / nseg);
+        const int i1 = (int)(((long)(s + 1) * (nd + 1)) / nseg);
         const long st = stride<D>(a);
-        Face<T> prev, fm;
+        Face<T> fm, fp, prev;
         // with the selector (single precision) the stencil stays in registers
         // and slides one cell per step: one new load per field instead of
         // five.  The fixed-scheme kernels reload it from cache; the window's
@@ -446,36 +486,39 @@ __global__ __launch_bounds__(256) void k_flux_yz(ArgsT<T> a, int nseg) {
         long cc = cidx(a, j, (D == 1) ? i0 : o2, (D == 1) ? o2 : i0);
         if constexpr (slide) {
             load_stencil<T, stencil_r<R>(), D>(a, cc, st, win);
-            recon_stencil<T, R, D>(a, cc, i0, win, fm, prev);
+            recon_stencil<T, R, D, true>(a, cc, i0, win, fm, fp);
         } else {
-            recon_at<T, R, D>(a, j, (D == 1) ? i0 : o2, (D == 1) ? o2 : i0, st, fm, prev);
+            recon_at<T, R, D, true>(a, j, (D == 1) ? i0 : o2, (D == 1) ? o2 : i0, st, fm, fp);
         }
         const T carry = (T)a.S->carry[D];
+        if constexpr (lds) keep_face(kept, fp);
+        else prev = fp;
 #pragma unroll 1
         for (int i = i0 + 1; i <= i1; ++i) {
-            int k = (D == 1) ? i : o2;
-            int l = (D == 1) ? o2 : i;
-            Face<T> fp;
+            const int k = (D == 1) ? i : o2;
+            const int l = (D == 1) ? o2 : i;
+            const long c = cc;
             cc += st;
             if constexpr (slide) {
                 slide_stencil<T, R, D>(a, cc, st, win);
-                recon_stencil<T, R, D>(a, cc, i, win, fm, fp);
+                recon_stencil<T, R, D, true>(a, cc, i, win, fm, fp);
             } else {
-                recon_at<T, R, D>(a, j, k, l, st, fm, fp);
+                recon_at<T, R, D, true>(a, j, k, l, st, fm, fp);
             }
-            int kk = (D == 1) ? i - 1 : k;
-            int ll = (D == 1) ? l : i - 1;
-            long c = cidx(a, j, kk, ll);
+            if constexpr (lds) {
+                prev = kept_face(kept);
+                keep_face(kept, fp);
+            }
             T bn = (T)a.Bin[D][c];
             Q<T> qL = to_q<T, D>(prev, bn), qR = to_q<T, D>(fm, bn);
             RiemannOut<T> o;
             riemann<T, D, S>(qL, qR, prev.eps, fm.eps, prev.cs, fm.cs, a.bn_mode, carry, o);
             store_face<T, D, S>(a, c, o, i == 1);
             if (o.ds) {
-                unsigned long long kk2 = serial_key<D>(a, j, kk, ll);
-                key = kk2 > key ? kk2 : key;
+                const unsigned long long kk = serial_key<D>(a, j, (D == 1) ? i - 1 : k, (D == 1) ? l : i - 1);
+                key = kk > key ? kk : key;
             }
-            prev = fp;
+            if constexpr (!lds) prev = fp;
         }
     }
     if constexpr (S == 3) {
@@ -510,8 +553,8 @@ __global__ __launch_bounds__(64) void k_carry(ArgsT<T> a) {
     }
     const long st = stride<D>(a);
     Face<T> lm, lp, rm, rp;
-    recon_at<T, R, D>(a, j, k, l, st, lm, lp);
-    recon_at<T, R, D>(a, j + (D == 0), k + (D == 1), l + (D == 2), st, rm, rp);
+    recon_at<T, R, D, false>(a, j, k, l, st, lm, lp);
+    recon_at<T, R, D, false>(a, j + (D == 0), k + (D == 1), l + (D == 2), st, rm, rp);
     T bn = (T)a.Bin[D][cidx(a, j, k, l)];
     Q<T> qL = to_q<T, D>(lp, bn), qR = to_q<T, D>(rm, bn);
     RiemannOut<T> o;

@@ -37,9 +37,10 @@ __device__ __forceinline__ float sqrtT(float a) { return __builtin_sqrtf(a); }
 // issue, and IEEE division is over half of their instructions: 11 per
 // quotient as the compiler expands it (two v_div_scale, v_rcp_f64 at a quarter
 // of the rate, five refining fma/mul, residual, v_div_fmas, v_div_fixup).
-// Den<double> forms the refined reciprocal once per denominator (5
-// instructions) and each quotient takes 4 more (product, residual, correction,
-// v_div_fixup): the compiler's own operations without the range scaling.  They
+// Den<double> forms the refined reciprocal once per denominator (4
+// instructions: the seed, its error e, e + e^2, and the cubic correction, in
+// place of two Newton steps) and each quotient takes 4 more (product, residual,
+// correction, v_div_fixup): the compiler's own without the range scaling.  They
 // give the same bits wherever scaling would not have acted: numerator 0 or
 // from 2^-969 up (below it the residual underflows), denominator and quotient
 // clear of the ends of the range.  Zeros, infinities and NaN are
@@ -59,7 +60,7 @@ __device__ __forceinline__ float sqrtT(float a) { return __builtin_sqrtf(a); }
 // speed.  Denominators here are densities, differences of signal speeds and
 // the like, from 2^-700 up or 0.  In single precision all of these are the
 // plain operators, which the FP32 unit turns into reciprocals that it shares.
-// (MI355X, FP64, HLLD + WENO-Z at 256^3: x sweep 1.92 -> 1.59 ms, y 2.70 ->
+// (MI355X, FP64, HLLD + WENO-Z at 256^3: x sweep 1.92 -> 1.58 ms, y 2.70 ->
 // 2.05, z 2.33 -> 1.95; HLLD + PPM at 128^3: x 0.162 -> 0.150 ms; HLL + MC at
 // 150 x 130 x 110: x 0.100 -> 0.091 ms.)
 template <class T> struct Den {
@@ -72,8 +73,8 @@ template <> struct Den<double> {
     double d, y;
     __device__ __forceinline__ explicit Den(double x) : d(x) {
         y = __builtin_amdgcn_rcp(x);
-        y = __builtin_fma(__builtin_fma(-x, y, 1.0), y, y);
-        y = __builtin_fma(__builtin_fma(-x, y, 1.0), y, y);
+        const double e = __builtin_fma(-x, y, 1.0);
+        y = __builtin_fma(__builtin_fma(e, e, e), y, y);
     }
     __device__ __forceinline__ double operator()(double n) const {
         const double q = n * y;

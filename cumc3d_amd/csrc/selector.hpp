@@ -73,8 +73,8 @@ __device__ __forceinline__ void sel_features(const ArgsT<W> &a, long c, long st,
 template <class W, int D>
 __device__ __forceinline__ int sel_label(const ArgsT<W> &a, long c, int i, long st, float thr_ppm, float thr_weno) {
     float wt[NW], ww[NW];
-    load_w<float>(a.ax[D].wsel[0] + (long)(i + 3) * NW, wt, 2);
-    load_w<float>(a.ax[D].wsel[2] + (long)(i + 3) * NW, ww, 10);
+    load_w<float, W, false>(a.ax[D].wsel[0], i, wt, 2);
+    load_w<float, W, false>(a.ax[D].wsel[2], i, ww, 10);
     float err = 0.0f;
 #pragma unroll
     for (int v = 0; v < 2; ++v) {
