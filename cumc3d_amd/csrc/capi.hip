@@ -628,6 +628,16 @@ int cumc3d_init(const cumc3d_desc *desc, cumc3d_ctx **out) {
         long v = atol(mt);
         if (v >= 1) x->march_threads = v;
     }
+    if (d.riemann == CUMC3D_HLLD && d.hlld_bn_mode == 2) {
+        size_t at[4] = {};
+        for (int D = 0; D < 3; ++D) {
+            int ns;
+            const dim3 g = sweep_grid(x, D, ns);
+            at[D + 1] = at[D] + (D < d.n_dim ? (size_t)g.x * g.y : 0);
+        }
+        if (hipMalloc(&x->slot[0], at[3] * sizeof(double2)) != hipSuccess) { cleanup(); return fail(CUMC3D_ENOMEM, "carry slots"); }
+        for (int D = 1; D < 3; ++D) x->slot[D] = x->slot[0] + at[D];
+    }
     if (d.riemann == CUMC3D_HLL) {
         if (hipMalloc(&x->stale, (size_t)3 * x->G) != hipSuccess) { cleanup(); return fail(CUMC3D_ENOMEM, "stale flags"); }
         if (hipMemset(x->stale, 0, (size_t)3 * x->G) != hipSuccess) { cleanup(); return fail(CUMC3D_EHIP, "memset"); }
@@ -1000,6 +1010,7 @@ int cumc3d_finalize(cumc3d_ctx *x) {
     if (x->wtab) hipFree(x->wtab);
     if (x->S) hipFree(x->S);
     if (x->stale) hipFree(x->stale);
+    if (x->slot[0]) hipFree(x->slot[0]);
     if (x->grav) hipFree(x->grav);
     if (x->ev_x) hipEventDestroy(x->ev_x);
     if (x->ev_m) hipEventDestroy(x->ev_m);

@@ -37,6 +37,7 @@ struct cumc3d_ctx {
     float *sel_w = nullptr, *sel_m = nullptr, *sel_v = nullptr;   // FP32 parameters + Adam moments
     unsigned short *sel_frag = nullptr;                            // BF16 MFMA fragments
     unsigned char *mask = nullptr;                                 // 3 x G class mask
+    double2 *slot[3] = {};                                          // HLLD: carry slots per sweep (one allocation, slot[0])
     unsigned char *stale = nullptr;                                // HLL: 3 x G unassigned-face flags
     const double *sph[10] = {};   // spherical tables in met (see ArgsT), null on other geometries
     float *samp_feat = nullptr;
@@ -277,6 +278,7 @@ template <class W> static ArgsT<W> make_args(cumc3d_ctx *x) {
     a.efl = x->floors[2];
     a.S = x->S;
     for (int d = 0; d < 3; ++d) a.mask[d] = x->mask ? x->mask + (size_t)d * x->G : nullptr;
+    for (int d = 0; d < 3; ++d) a.slot[d] = x->slot[d];
     for (int d = 0; d < 3; ++d) a.stale[d] = x->stale ? x->stale + (size_t)d * x->G : nullptr;
     a.dcb = x->sph[0]; a.dcb3 = x->sph[1]; a.xbar = x->sph[2]; a.gsrc = x->sph[3]; a.hbx = x->sph[4];
     a.sinf = x->sph[5]; a.dcose = x->sph[6]; a.cot = x->sph[7]; a.hby = x->sph[8]; a.sine = x->sph[9];
@@ -304,27 +306,26 @@ static int nseg_for(const cumc3d_ctx *x, int nx, int na, int nd) {
 // ---------------------------------------------------------------------------
 // flux dispatch over (reconstruction, Riemann solver)
 // ---------------------------------------------------------------------------
+// Grid of the sweep along D: x by waves of 63 interfaces (k_flux_x), y and z by
+// planes across the sweep axis and march segments (k_flux_yz).
+static dim3 sweep_grid(const cumc3d_ctx *x, int D, int &nseg) {
+    nseg = 1;
+    if (D == 0) {
+        const long waves = ((long)(x->nx + 2) * x->ny * x->nz + 62) / 63 + 1;
+        return dim3((unsigned)((waves * 64 + 255) / 256));
+    }
+    const int na = D == 1 ? x->nz : x->ny, nd = D == 1 ? x->ny : x->nz;
+    nseg = nseg_for(x, x->nx, na, nd);
+    return dim3(nblk((long)x->nx * na), nseg);
+}
+
 template <class W, int R, int S>
 static void launch_sweep_rs(cumc3d_ctx *x, const ArgsT<W> &a, int D, hipStream_t st) {
-    if (D == 0) {
-        long waves = ((long)(x->nx + 2) * x->ny * x->nz + 62) / 63 + 1;
-        unsigned grid = (unsigned)((waves * 64 + 255) / 256);
-        hipLaunchKernelGGL((k_flux_x<W, R, S>), dim3(grid), dim3(256), 0, st, a);
-        if (S == 3 && a.bn_mode == 2)
-            hipLaunchKernelGGL((k_carry<W, R, 0>), dim3(1), dim3(64), 0, st, a);
-    } else if (D == 1) {
-        int ns = nseg_for(x, x->nx, x->nz, x->ny);
-        const dim3 grid(nblk((long)x->nx * x->nz), ns);
-        hipLaunchKernelGGL((k_flux_yz<W, R, S, 1>), grid, dim3(256), 0, st, a, ns);
-        if (S == 3 && a.bn_mode == 2)
-            hipLaunchKernelGGL((k_carry<W, R, 1>), dim3(1), dim3(64), 0, st, a);
-    } else {
-        int ns = nseg_for(x, x->nx, x->ny, x->nz);
-        const dim3 grid(nblk((long)x->nx * x->ny), ns);
-        hipLaunchKernelGGL((k_flux_yz<W, R, S, 2>), grid, dim3(256), 0, st, a, ns);
-        if (S == 3 && a.bn_mode == 2)
-            hipLaunchKernelGGL((k_carry<W, R, 2>), dim3(1), dim3(64), 0, st, a);
-    }
+    int ns;
+    const dim3 grid = sweep_grid(x, D, ns);
+    if (D == 0) hipLaunchKernelGGL((k_flux_x<W, R, S>), grid, dim3(256), 0, st, a);
+    else if (D == 1) hipLaunchKernelGGL((k_flux_yz<W, R, S, 1>), grid, dim3(256), 0, st, a, ns);
+    else hipLaunchKernelGGL((k_flux_yz<W, R, S, 2>), grid, dim3(256), 0, st, a, ns);
 }
 
 template <class W, int R>
@@ -389,8 +390,9 @@ template <class W> static void sweeps_t(cumc3d_ctx *x, const ArgsT<W> &a, hipStr
     mark(2);
     if (x->d.n_dim > 2) launch_sweep(x, a, 2, st);
     mark(3);
-    hipLaunchKernelGGL(k_emf_prep<W>, dim3(nblk(emf_prep_count(a))), dim3(256), 0, st, a);
-    hipLaunchKernelGGL(k_edge<W>, dim3(nblk((long)(x->nx + 1) * (x->ny + 1) * (x->nz + 1))), dim3(256), 0, st, a);
+    const dim3 ge(nblk((long)(x->nx + 1) * (x->ny + 1) * (x->nz + 1)));
+    if (x->d.n_dim == 3) hipLaunchKernelGGL((k_edge<W, true>), ge, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((k_edge<W, false>), ge, dim3(256), 0, st, a);
     if (a.fixpole) hipLaunchKernelGGL(k_fixpole<W>, dim3(2 * x->nx), dim3(64), 0, st, a);
     mark(4);
 }

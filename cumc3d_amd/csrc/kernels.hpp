@@ -6,7 +6,7 @@
 // the variable index moved out to the slowest position.
 //
 // Per stage: x/y/z interface fluxes (reconstruction + face states + Riemann
-// solver), the HLLD carry fix-up per sweep, edge EMFs, the fused update
+// solver), edge EMFs, the fused update
 // (flux divergence, sources, RK combine, CT, cons->prim->cons, floors, EOS,
 // CFL minimum in stage 3) and the ghost fill.
 #pragma once
@@ -23,8 +23,10 @@ struct DevScalars {
     double t;                         // global_time
     double total_time;
     unsigned long long dtmin_bits;    // CFL min (bit pattern of a positive double)
-    double carry[3];                  // HLLD usstar carried per field component (x,y,z)
-    unsigned long long carry_key;     // max serial key of the sweep's double-star interfaces (0: none)
+    double carry[3];                  // HLLD usstar carried per field component (x,y,z) into this stage
+    // per sweep of this stage: serial key of its last double-star interface
+    // (high word; 0: none) and the block that holds it (low word)
+    unsigned long long carry_key[3];
     int nstep;
     int active;                       // 0 once global_time >= total_time: stage kernels exit
     int nonfinite;                    // set when a cell's CFL time step is NaN or not positive
@@ -87,6 +89,9 @@ template <class W> struct ArgsT {
     // collapsar: potential over the ghosted box, atmosphere prim_a(irho:ivz) and eps_a
     const double *phi;
     double pa[4], eps_a;
+    // HLLD carry: per sweep and block, the transverse field of the double-star
+    // state of the block's last such interface (see carried())
+    double2 *slot[3];
     // SPATIAL alone (k_update<0>): l_rk(1:8) in the host layout, var fastest
     double *lrk;
 };
@@ -150,12 +155,13 @@ template <class A> __device__ __forceinline__ double gsign(const A &a, int axis,
 
 // Serial position of interface (j,k,l) in the reference's Riemann loop
 // (rsolver_module.f90:596-598: l outer, j inner; the sweep axis starts at 0,
-// the others at 1), plus one.
+// the others at 1), plus one.  Below 2^30: a field stays below 4 GiB.
 template <int D, class A>
-__device__ __forceinline__ unsigned long long serial_key(const A &a, int j, int k, int l) {
-    if constexpr (D == 0) return ((unsigned long long)(l - 1) * a.ny + (k - 1)) * (a.nx + 1) + j + 1;
-    else if constexpr (D == 1) return ((unsigned long long)(l - 1) * (a.ny + 1) + k) * a.nx + (j - 1) + 1;
-    else return ((unsigned long long)l * a.ny + (k - 1)) * a.nx + (j - 1) + 1;
+__device__ __forceinline__ unsigned serial_key(const A &a, int j, int k, int l) {
+    const unsigned nx = a.nx, ny = a.ny;
+    if constexpr (D == 0) return ((unsigned)(l - 1) * ny + (k - 1)) * (nx + 1) + j + 1;
+    else if constexpr (D == 1) return ((unsigned)(l - 1) * (ny + 1) + k) * nx + (j - 1) + 1;
+    else return ((unsigned)l * ny + (k - 1)) * nx + (j - 1) + 1;
 }
 
 // 7-variable stencil of cell c along D: rho, vx, vy, vz, p and the two
@@ -369,13 +375,71 @@ __device__ __forceinline__ unsigned long long block_max_u64(unsigned long long v
     return v;
 }
 
+// The HLLD carry.  The serial reference leaves the transverse field of the
+// last double-star interface behind in usstarL/usstarR and reads it back as
+// usstar(ibn) in later sweeps (rsolver_module.f90:704-741).  Every block of a
+// sweep finds its last double-star interface in the reference's loop order
+// (key: its serial position), writes the two components to the block's slot
+// and folds (key, block) into the sweep's maximum; the sweeps after it pick
+// the value up from there (carried()) and k_edge, which follows the stage's
+// sweeps, folds the three into S->carry.  No kernel of its own runs for it: the
+// re-solve of the one interface by a single thread took 5-18 us after every
+// sweep, a sixth of the step on small grids.
+// A block whose key does not exceed the maximum folded so far skips its
+// atomic (its slot is then never read).
+template <class T>
+__device__ __forceinline__ void fold_carry(DevScalars *S, double2 *slot, int sweep, unsigned serial, const T left[][256]) {
+    const unsigned block = blockIdx.y * gridDim.x + blockIdx.x;
+    const unsigned long long key = (unsigned long long)serial << 32 | block;
+    __shared__ unsigned long long last;
+    const unsigned long long m = block_max_u64(serial ? key : 0ULL);
+    if (threadIdx.x == 0) last = m;
+    __syncthreads();
+    if (serial && key == last &&
+        key > __hip_atomic_load(&S->carry_key[sweep], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+        slot[block] = make_double2(left[0][threadIdx.x], left[1][threadIdx.x]);
+        atomicMax(&S->carry_key[sweep], key);
+    }
+}
+
+// The carried value of component D for the sweep along D: a sweep along d
+// leaves component d+1 in the slot's x and d+2 in its y.
+template <int D, class A> __device__ __forceinline__ double carried(const A &a) {
+    const DevScalars *S = a.S;
+    if constexpr (D == 1) {
+        const unsigned long long k0 = S->carry_key[0];
+        if (k0) return a.slot[0][(unsigned)k0].x;
+    } else if constexpr (D == 2) {
+        const unsigned long long k0 = S->carry_key[0], k1 = S->carry_key[1];
+        if (k1) return a.slot[1][(unsigned)k1].x;
+        if (k0) return a.slot[0][(unsigned)k0].y;
+    }
+    return S->carry[D];
+}
+
+// After the sweeps of a stage (one thread): the value each component carries
+// into the next stage, and no double-star interface yet.
+template <class A> __device__ __forceinline__ void settle_carry(const A &a) {
+    double c[3] = {a.S->carry[0], a.S->carry[1], a.S->carry[2]};
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const unsigned long long k = a.S->carry_key[d];
+        if (!k) continue;
+        const double2 v = a.slot[d][(unsigned)k];
+        c[(d + 1) % 3] = v.x;
+        c[(d + 2) % 3] = v.y;
+        a.S->carry_key[d] = 0;
+    }
+    for (int d = 0; d < 3; ++d) a.S->carry[d] = c[d];
+}
+
 // x sweep.  The (nx+2) cells j=0..nx+1 of every row are laid end to end; each
 // 64-lane wave reconstructs 64 consecutive cells and solves the 63 interfaces
 // between them, taking the right neighbour's left face with a lane shuffle.
 // Waves overlap by one cell, so every cell is reconstructed about 64/63 times.
 // Blocks take the rows from the last to the first: the first blocks hold the
-// largest serial keys of the HLLD carry, and a later block whose key does not
-// exceed the value already folded skips its atomic.  (In order, nearly every
+// largest serial keys of the HLLD carry, so that later blocks skip their
+// atomic (fold_carry).  (In order, nearly every
 // one of the ~68k blocks of a 256^3 sweep with many double-star interfaces
 // raised the maximum, and the atomics on the one address serialised: FP32
 // TVD-MC x sweep 0.79 ms against 0.39 ms for the z sweep on turbulence.)
@@ -412,36 +476,36 @@ void k_flux_x(ArgsT<T> a) {
     nm.bt2 = __shfl_down(fm.bt2, 1, 64);
     nm.eps = __shfl_down(fm.eps, 1, 64);
     nm.cs = __shfl_down(fm.cs, 1, 64);
-    unsigned long long key = 0;
+    unsigned serial = 0;
+    __shared__ T left[S == 3 ? 2 : 1][256];   // carry of the thread's interface
     if (live && lane < 63 && j <= a.nx && g + 1 < gtot) {
         long c = cidx(a, j, k, l);
         T bn = (T)a.Bin[0][c];
         Q<T> qL = to_q<T, 0>(fp, bn), qR = to_q<T, 0>(nm, bn);
         RiemannOut<T> o;
-        riemann<T, 0, S>(qL, qR, fp.eps, nm.eps, fp.cs, nm.cs, a.bn_mode, (T)a.S->carry[0], o);
+        riemann<T, 0, S>(qL, qR, fp.eps, nm.eps, fp.cs, nm.cs, a.bn_mode, S == 3 ? (T)carried<0>(a) : T(0), o);
         store_face<T, 0, S>(a, c, o, j == 0);
-        if (o.ds) key = serial_key<0>(a, j, k, l);
+        if (S == 3 && a.bn_mode == 2 && o.ds) {
+            serial = serial_key<0>(a, j, k, l);
+            left[0][threadIdx.x] = o.uss_t1;
+            left[1][threadIdx.x] = o.uss_t2;
+        }
     }
     if constexpr (S == 3) {
-        if (a.bn_mode == 2) {
-            key = block_max_u64(key);
-            if (threadIdx.x == 0 && key &&
-                key > __hip_atomic_load(&a.S->carry_key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-                atomicMax(&a.S->carry_key, key);
-        }
+        if (a.bn_mode == 2) fold_carry(a.S, a.slot[0], 0, serial, left);
     }
 }
 
 // Where a marching thread keeps the right face of the cell behind it: LDS (its
 // own column of the block's array) or registers.  The memory clobber stops the
 // compiler from carrying the slot in registers across the loop.
-template <class T> __device__ __forceinline__ void keep_face(T kept[9][256], const Face<T> &f) {
+template <class T> __device__ __forceinline__ void keep_face(T kept[][256], const Face<T> &f) {
     const int t = threadIdx.x;
     kept[0][t] = f.rho; kept[1][t] = f.v[0]; kept[2][t] = f.v[1]; kept[3][t] = f.v[2]; kept[4][t] = f.p;
     kept[5][t] = f.bt1; kept[6][t] = f.bt2; kept[7][t] = f.eps; kept[8][t] = f.cs;
     __asm__ volatile("" ::: "memory");
 }
-template <class T> __device__ __forceinline__ Face<T> kept_face(const T kept[9][256]) {
+template <class T> __device__ __forceinline__ Face<T> kept_face(const T kept[][256]) {
     const int t = threadIdx.x;
     return {kept[0][t], {kept[1][t], kept[2][t], kept[3][t]}, kept[4][t], kept[5][t], kept[6][t], kept[7][t], kept[8][t]};
 }
@@ -453,21 +517,20 @@ template <class T> __device__ __forceinline__ Face<T> kept_face(const T kept[9][
 // cell's right face.
 // What bounds it: VALU issue, given waves to issue from.  With the kept face
 // in registers the FP64 march needed 168 to 256 VGPRs and up to 78 AGPRs (one
-// or two waves per SIMD); in LDS it needs at most 186 (three waves but for
-// HLL + WENO-Z), and the selector's 123 instead of 125 with fewer copies.
-// Measured at 256^3, y / z sweep: FP64 HLLD + WENO-Z 2.05 / 1.95 -> 1.64 /
-// 1.65 ms, FP32 selector 0.426 / 0.430 -> 0.405 / 0.409 ms.  The FP32 fixed
-// schemes keep it in registers: from LDS, TVD-MC took 0.360 against 0.353 ms
-// and PPM 0.495 against 0.474 ms.
+// or two waves per SIMD); in LDS it fits three.  Measured at 256^3, y / z sweep,
+// HLLD + WENO-Z: 2.05 / 1.95 -> 1.56 / 1.56 ms.  In single precision the face
+// stays in registers for the fixed schemes: from LDS, TVD-MC took 0.360 against
+// 0.353 ms and PPM 0.495 against 0.474 ms (the selector 0.400 against 0.467).
 template <class T, int R, int S, int D>
-__global__ __launch_bounds__(256) void k_flux_yz(ArgsT<T> a, int nseg) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 3 : 1))) void k_flux_yz(ArgsT<T> a, int nseg) {
     if (!a.S->active) return;
     const unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
     const int na = (D == 1) ? a.nz : a.ny;    // the other transverse axis
     const int nd = (D == 1) ? a.ny : a.nz;    // sweep axis
-    unsigned long long key = 0;
+    unsigned serial = 0;
     constexpr bool lds = sizeof(T) == 8 || R == RSEL;
     __shared__ T kept[lds ? 9 : 1][256];
+    __shared__ T left[S == 3 ? 2 : 1][256];   // carry of the thread's last double-star interface
     if (t < (unsigned)a.nx * (unsigned)na) {
         const int o2 = 1 + (int)(t / (unsigned)a.nx);
         const int j = 1 + (int)(t - (unsigned)(o2 - 1) * (unsigned)a.nx);
@@ -490,9 +553,10 @@ __global__ __launch_bounds__(256) void k_flux_yz(ArgsT<T> a, int nseg) {
         } else {
             recon_at<T, R, D, true>(a, j, (D == 1) ? i0 : o2, (D == 1) ? o2 : i0, st, fm, fp);
         }
-        const T carry = (T)a.S->carry[D];
+        const T carry = S == 3 ? (T)carried<D>(a) : T(0);
         if constexpr (lds) keep_face(kept, fp);
         else prev = fp;
+        int dsi = 0;   // the march's last double-star interface lies below cell dsi
 #pragma unroll 1
         for (int i = i0 + 1; i <= i1; ++i) {
             const int k = (D == 1) ? i : o2;
@@ -514,67 +578,23 @@ __global__ __launch_bounds__(256) void k_flux_yz(ArgsT<T> a, int nseg) {
             RiemannOut<T> o;
             riemann<T, D, S>(qL, qR, prev.eps, fm.eps, prev.cs, fm.cs, a.bn_mode, carry, o);
             store_face<T, D, S>(a, c, o, i == 1);
-            if (o.ds) {
-                const unsigned long long kk = serial_key<D>(a, j, (D == 1) ? i - 1 : k, (D == 1) ? l : i - 1);
-                key = kk > key ? kk : key;
+            if (S == 3 && a.bn_mode == 2 && o.ds) {   // the serial order grows along the march
+                dsi = i;
+                left[0][threadIdx.x] = o.uss_t1;
+                left[1][threadIdx.x] = o.uss_t2;
             }
             if constexpr (!lds) prev = fp;
         }
+        if (dsi > 0) serial = serial_key<D>(a, j, (D == 1) ? dsi - 1 : o2, (D == 1) ? o2 : dsi - 1);
     }
     if constexpr (S == 3) {
-        if (a.bn_mode == 2) {
-            key = block_max_u64(key);
-            if (threadIdx.x == 0 && key) atomicMax(&a.S->carry_key, key);
-        }
+        if (a.bn_mode == 2) fold_carry(a.S, a.slot[D], D, serial, left);
     }
-}
-
-// After a sweep: find the last double-star interface in the reference's serial
-// loop order and recompute its double-star transverse field, which the serial
-// reference leaves behind in usstarL/usstarR and reads back as usstar(ibn) in
-// later sweeps (rsolver_module.f90:704-741).
-template <class T, int R, int D>
-__global__ __launch_bounds__(64) void k_carry(ArgsT<T> a) {
-    if (!a.S->active || threadIdx.x != 0) return;
-    const unsigned long long key = a.S->carry_key;
-    a.S->carry_key = 0;     // the next sweep starts from no double-star interface
-    if (key == 0) return;
-    unsigned long long q = key - 1;
-    int j, k, l;
-    if constexpr (D == 0) {
-        j = (int)(q % (a.nx + 1)); q /= (a.nx + 1);
-        k = 1 + (int)(q % a.ny); l = 1 + (int)(q / a.ny);
-    } else if constexpr (D == 1) {
-        j = 1 + (int)(q % a.nx); q /= a.nx;
-        k = (int)(q % (a.ny + 1)); l = 1 + (int)(q / (a.ny + 1));
-    } else {
-        j = 1 + (int)(q % a.nx); q /= a.nx;
-        k = 1 + (int)(q % a.ny); l = (int)(q / a.ny);
-    }
-    const long st = stride<D>(a);
-    Face<T> lm, lp, rm, rp;
-    recon_at<T, R, D, false>(a, j, k, l, st, lm, lp);
-    recon_at<T, R, D, false>(a, j + (D == 0), k + (D == 1), l + (D == 2), st, rm, rp);
-    T bn = (T)a.Bin[D][cidx(a, j, k, l)];
-    Q<T> qL = to_q<T, D>(lp, bn), qR = to_q<T, D>(rm, bn);
-    RiemannOut<T> o;
-    riemann<T, D, 3>(qL, qR, lp.eps, rm.eps, lp.cs, rm.cs, a.bn_mode, (T)a.S->carry[D], o);
-    a.S->carry[(D + 1) % 3] = (double)o.uss_t1;
-    a.S->carry[(D + 2) % 3] = (double)o.uss_t2;
 }
 
 // ---------------------------------------------------------------------------
 // constrained transport: edge EMFs (flux_ct, mhd_module.f90:310-426)
 // ---------------------------------------------------------------------------
-
-// cell-centred EMF -v x B of an interior cell (mhd_module.f90:316-318)
-template <int E, class W> __device__ __forceinline__ W ecell_raw(const ArgsT<W> &a, long c) {
-    W vx = a.P[1][c], vy = a.P[2][c], vz = a.P[3][c];
-    W bx = a.Bc[0][c], by = a.Bc[1][c], bz = a.Bc[2][c];
-    if constexpr (E == 0) return vz * by - vy * bz;
-    else if constexpr (E == 1) return vx * bz - vz * bx;
-    else return vy * bx - vx * by;
-}
 
 // Store the cell EMFs of cell c from its velocity and cell-centred field
 // (times a parity factor per component for mapped ghost cells).
@@ -586,127 +606,77 @@ __device__ __forceinline__ void cell_emf(const ArgsT<W> &a, long c, W vx, W vy, 
     a.Ec[2][c] = s2 * (vy * bx - vx * by);
 }
 
-// ecell after BOUNDARY_EFIELD (mhd_module.f90:478-840): ghost cells take the
-// mapped interior value times the parity factors of component E.
-template <int E, class W> __device__ __forceinline__ W ecell_at(const ArgsT<W> &a, int j, int k, int l) {
-    int sx, sy, sz;
-    int jj = gmap(j, a.nx, a.bc[0], a.bc[1], sx);
-    int kk = gmap(k, a.ny, a.bc[2], a.bc[3], sy);
-    int ll = gmap(l, a.nz, a.bc[4], a.bc[5], sz);
-    W s = (W)(gsign(a, 0, sx, 9 + E) * gsign(a, 1, sy, 9 + E) * gsign(a, 2, sz, 9 + E));
-    W v = ecell_raw<E>(a, cidx(a, jj, kk, ll));
-    return (sx < 0 && sy < 0 && sz < 0) ? v : s * v;
+// Where the edge stencil's cell indices i and i+1 (i = 0..n) along an axis
+// read face EMFs (BOUNDARY_EFIELD, mhd_module.f90:478-840): the offset to the
+// mapped interior cell and the parity of EMF components E1 and E2, for i and i+1.
+template <class W> struct EdgeAxis {
+    long at[2];
+    W s1[2], s2[2];
+};
+template <int X, int E1, int E2, class W>
+__device__ __forceinline__ EdgeAxis<W> edge_axis(const ArgsT<W> &a, int i) {
+    const int n = X == 0 ? a.nx : (X == 1 ? a.ny : a.nz);
+    const long st = X == 0 ? 1L : (X == 1 ? a.NX : a.NX * a.NY);
+    const long lo = (a.bc[2 * X] == 0 ? n : 1) * st, hi = (a.bc[2 * X + 1] == 0 ? -n : -1) * st;
+    EdgeAxis<W> r;
+    r.at[0] = i == 0 ? lo : 0;
+    r.at[1] = i == n ? st + hi : st;
+    r.s1[0] = i == 0 ? (W)gsign(a, X, 0, 9 + E1) : W(1);
+    r.s1[1] = i == n ? (W)gsign(a, X, 1, 9 + E1) : W(1);
+    r.s2[0] = i == 0 ? (W)gsign(a, X, 0, 9 + E2) : W(1);
+    r.s2[1] = i == n ? (W)gsign(a, X, 1, 9 + E2) : W(1);
+    return r;
 }
 
-// Face EMF eface of component E at faces normal to D, after the 1D/2D fill
-// (mhd_module.f90:328-356) and BOUNDARY_EFIELD: face index along D is real,
-// the two cell-centred axes are ghost-mapped.
-template <int E, int D, class W> __device__ __forceinline__ W eface_at(const ArgsT<W> &a, int j, int k, int l) {
-    int sx = -1, sy = -1, sz = -1;
-    if constexpr (D != 0) j = gmap(j, a.nx, a.bc[0], a.bc[1], sx);
-    if constexpr (D != 1) k = gmap(k, a.ny, a.bc[2], a.bc[3], sy);
-    if constexpr (D != 2) l = gmap(l, a.nz, a.bc[4], a.bc[5], sz);
-    W v;
-    if (D < a.ndim) {
-        constexpr int slot = (D == 0) ? (E == 1 ? 5 : 6) : (D == 1 ? (E == 0 ? 5 : 6) : (E == 0 ? 5 : 6));
-        v = a.F[D][slot][cidx(a, j, k, l)];
-    } else {
-        if constexpr (D == 0) j = 1;
-        else if constexpr (D == 1) k = 1;
-        else l = 1;
-        v = ecell_raw<E>(a, cidx(a, j, k, l));
-    }
-    if (sx < 0 && sy < 0 && sz < 0) return v;
-    return (W)(gsign(a, 0, sx, 9 + E) * gsign(a, 1, sy, 9 + E) * gsign(a, 2, sz, 9 + E)) * v;
-}
-
-// Face EMFs on the cells 0..n+1 the edge stencil reads (flux_ct,
-// mhd_module.f90:310-360, ghosts mapped as in BOUNDARY_EFIELD): the ghost rows
-// along their two cell-centred axes plus the faces of inactive directions
-// (1D/2D fill).  The cell EMFs (ecell) are stored by the update for interior
-// cells and by the ghost fill (mapped) for ghost cells.
-// Cells of the (n+2)^3 box 0..n+1 the face-EMF fill visits: in 3D only its
-// outer shell (a ghost index on some axis), in 1D/2D every cell (the
-// inactive directions' faces are filled everywhere).
-template <class A> __host__ __device__ __forceinline__ long emf_prep_count(const A &a) {
-    const long m = (long)(a.nx + 2) * (a.ny + 2) * (a.nz + 2);
-    return a.ndim == 3 ? m - (long)a.nx * a.ny * a.nz : m;
-}
-
-template <class W> __global__ __launch_bounds__(256) void k_emf_prep(ArgsT<W> a) {
+// Edge EMFs (flux_ct, mhd_module.f90:414-423) on the edges the CT update reads:
+// efield_x for j=1..nx, efield_y for k=1..ny, efield_z for l=1..nz (0..n along
+// the other axes), from the face EMFs of the sweeps and the cell EMFs that the
+// update (interior) and the ghost fill (mapped ghosts) stored.  Memory bounds
+// it; each face EMF is a ghost along at most one axis, and mapping that index
+// here costs a few instructions, where a kernel that filled the ghost rows
+// first took 7-23 us a stage.  In 1D and 2D (DIM3 false) the faces of an
+// inactive direction hold the cell EMF at index 1 along it (mhd_module.f90:328-356),
+// mapped along the other axes by the ghost fill.
+template <class W, bool DIM3> __global__ __launch_bounds__(256) void k_edge(ArgsT<W> a) {
     if (!a.S->active) return;
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= emf_prep_count(a)) return;
-    int j, k, l;
-    if (a.ndim == 3) {
-        // shell of the box: the two z planes, the two y rows of each inner
-        // plane, the two x cells of each inner row
-        const long n0 = a.nx + 2, n1 = a.ny + 2, pz = 2 * n0 * n1, py = 2 * n0 * (long)a.nz;
-        long q = t;
-        if (q < pz) {
-            l = (q / (n0 * n1)) == 0 ? 0 : a.nz + 1;
-            k = (int)((q % (n0 * n1)) / n0);
-            j = (int)(q % n0);
-        } else if (q < pz + py) {
-            q -= pz;
-            l = 1 + (int)(q / (2 * n0));
-            k = ((q % (2 * n0)) / n0) == 0 ? 0 : a.ny + 1;
-            j = (int)(q % n0);
-        } else {
-            q -= pz + py;
-            l = 1 + (int)(q / (2L * a.ny));
-            k = 1 + (int)((q % (2L * a.ny)) / 2);
-            j = (q % 2) == 0 ? 0 : a.nx + 1;
-        }
-    } else {
-        const long n0 = a.nx + 2, n1 = a.ny + 2;
-        j = (int)(t % n0);
-        k = (int)((t / n0) % n1);
-        l = (int)(t / (n0 * n1));
-    }
-    const long c = cidx(a, j, k, l);
-    const bool gx = j < 1 || j > a.nx, gy = k < 1 || k > a.ny, gz = l < 1 || l > a.nz;
-    // x faces (face index j <= nx), cell axes y, z
-    if (j <= a.nx && (a.ndim < 1 || gy || gz)) {
-        a.F[0][5][c] = eface_at<1, 0>(a, j, k, l);
-        a.F[0][6][c] = eface_at<2, 0>(a, j, k, l);
-    }
-    if (k <= a.ny && (a.ndim < 2 || gx || gz)) {
-        a.F[1][5][c] = eface_at<0, 1>(a, j, k, l);
-        a.F[1][6][c] = eface_at<2, 1>(a, j, k, l);
-    }
-    if (l <= a.nz && (a.ndim < 3 || gx || gy)) {
-        a.F[2][5][c] = eface_at<0, 2>(a, j, k, l);
-        a.F[2][6][c] = eface_at<1, 2>(a, j, k, l);
-    }
-}
-
-// Edge EMFs (mhd_module.f90:414-423) on the edges the CT update reads:
-// efield_x for j=1..nx, efield_y for k=1..ny, efield_z for l=1..nz
-// (0..n along the other axes), from the arrays k_emf_prep completed.
-template <class W> __global__ __launch_bounds__(256) void k_edge(ArgsT<W> a) {
-    if (!a.S->active) return;
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long n1 = a.nx + 1, n2 = a.ny + 1;
-    if (t >= n1 * n2 * (a.nz + 1)) return;
-    const int j = (int)(t % n1), k = (int)((t / n1) % n2), l = (int)(t / (n1 * n2));
+    const unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t == 0 && a.slot[0]) settle_carry(a);
+    const unsigned n1 = a.nx + 1, n2 = a.ny + 1;
+    if (t >= n1 * n2 * (unsigned)(a.nz + 1)) return;
+    const unsigned row = t / n1;
+    const int j = (int)(t - row * n1), l = (int)(row / n2), k = (int)(row - l * n2);
     const long c = cidx(a, j, k, l), sy = a.NX, sz = a.NX * a.NY;
     const W *ex = a.Ec[0], *ey = a.Ec[1], *ez = a.Ec[2];
     const W h = W(0.50), q = W(0.25);
+    const EdgeAxis<W> X = edge_axis<0, 1, 2>(a, j), Y = edge_axis<1, 0, 2>(a, k), Z = edge_axis<2, 0, 1>(a, l);
+    // the four face EMFs around an edge, two per face direction
+    const auto pair = [&](int D, const W *f, const W *cell, int id, long st, const EdgeAxis<W> &A, const W s[2], W v[2],
+                          long step) {
+        if (DIM3 || D < a.ndim) {
+            v[0] = s[0] * f[c + A.at[0]];
+            v[1] = s[1] * f[c + A.at[1]];
+        } else {
+            v[0] = cell[c + (1 - id) * st];
+            v[1] = cell[c + (1 - id) * st + step];
+        }
+    };
     // the three EMFs are formed before any is stored, so that all their loads
     // are in flight together
-    W e0 = W(0), e1 = W(0), e2 = W(0);
+    W e0 = W(0), e1 = W(0), e2 = W(0), u[2], v[2];
     if (j >= 1) {
-        const W *fxy = a.F[1][5], *fxz = a.F[2][5];
-        e0 = h * (fxy[c] + fxy[c + sz] + fxz[c] + fxz[c + sy]) - q * (ex[c] + ex[c + sz] + ex[c + sy] + ex[c + sy + sz]);
+        pair(1, a.F[1][5], ex, k, sy, Z, Z.s1, u, sz);
+        pair(2, a.F[2][5], ex, l, sz, Y, Y.s1, v, sy);
+        e0 = h * (u[0] + u[1] + v[0] + v[1]) - q * (ex[c] + ex[c + sz] + ex[c + sy] + ex[c + sy + sz]);
     }
     if (k >= 1) {
-        const W *fyx = a.F[0][5], *fyz = a.F[2][6];
-        e1 = h * (fyx[c] + fyx[c + sz] + fyz[c] + fyz[c + 1]) - q * (ey[c] + ey[c + sz] + ey[c + 1] + ey[c + 1 + sz]);
+        pair(0, a.F[0][5], ey, j, 1, Z, Z.s2, u, sz);
+        pair(2, a.F[2][6], ey, l, sz, X, X.s1, v, 1);
+        e1 = h * (u[0] + u[1] + v[0] + v[1]) - q * (ey[c] + ey[c + sz] + ey[c + 1] + ey[c + 1 + sz]);
     }
     if (l >= 1) {
-        const W *fzx = a.F[0][6], *fzy = a.F[1][6];
-        e2 = h * (fzx[c] + fzx[c + sy] + fzy[c] + fzy[c + 1]) - q * (ez[c] + ez[c + sy] + ez[c + 1] + ez[c + 1 + sy]);
+        pair(0, a.F[0][6], ez, j, 1, Y, Y.s2, u, sy);
+        pair(1, a.F[1][6], ez, k, sy, X, X.s2, v, 1);
+        e2 = h * (u[0] + u[1] + v[0] + v[1]) - q * (ez[c] + ez[c + sy] + ez[c + 1] + ez[c + 1 + sy]);
     }
     if (j >= 1) a.E[0][c] = e0;
     if (k >= 1) a.E[1][c] = e1;
