@@ -225,11 +225,17 @@ static SorArgs sor_args(cumc3d_ctx *x) {
     a.rout = x->sor_phi[1][0];
     a.bout = x->sor_phi[1][1];
     a.rho_in = x->sor_rho;
-    a.a2 = x->sor_a2; a.e2 = x->sor_e2; a.zpm = x->sor_z[0]; a.zpc = x->sor_z[1]; a.zcm = x->sor_z[2];
+    a.a2 = x->sor_a2; a.e2 = x->sor_e2;
+    for (int i = 0; i < 3; ++i) {
+        a.z[i] = x->sor_z[i];
+        a.iz[i] = x->sor_z[3 + i];
+    }
     a.ajp1 = x->ajp1; a.ajm1 = x->ajm1; a.bkp1 = x->bkp1; a.bkm1 = x->bkm1;
     a.part_nan = x->part_nan;
     a.part_max = x->part_max;
     a.nblk = x->sor_nblk;
+    a.runs = x->sor_nblk / x->nz;
+    a.items = a.runs * 2 * (int)nblk(x->nz, 4);
     a.relax_max = x->grav_p.relax_max;
     a.pa = x->grav_p.prim_a[0];
     a.omega = x->grav_p.omega;
@@ -257,9 +263,8 @@ static int sor_solve(cumc3d_ctx *x, bool zero_guess) {
     SorArgs a = sor_args(x);
     hipLaunchKernelGGL(k_sor_rho, dim3(nblk((long)x->nx * x->ny), x->nz), dim3(256), 0, st, a,
                        (const double *)x->P[0], x->sor_rho);
-    const long hx = (x->nx + 1) / 2;
-    // red: one more block column, whose block (0, 0) decides the previous pair
-    const dim3 gr(nblk(hx * x->ny) + 1, x->nz), gb(nblk(hx * x->ny, SOR_SLOTS), x->nz);
+    // red: eight more blocks, the first of which decides the previous pair
+    const dim3 gb(8 * nblk(a.items, 8)), gr(8 + gb.x);
     const dim3 gc(nblk((long)x->nx * x->ny), x->nz);
     hipLaunchKernelGGL(k_sor_copy, gc, dim3(256), 0, st, a, x->phi, x->sor_phi[0][0], x->sor_phi[0][1], 1);
     long queued = 0;
@@ -519,16 +524,16 @@ int cumc3d_init(const cumc3d_desc *desc, cumc3d_ctx **out) {
     // from which the kernels form them with poisson_coef's divisions
     // (gravity.hpp); then room for rho_in, split by colour
     std::vector<double> pc;
-    long pco[10] = {};
+    long pco[13] = {};
     if (d.model == CUMC3D_MODEL_COLLAPSAR) {
         const int nx = d.nx, ny = d.ny, nz = d.nz;
         const long nb = (long)(nx + 1) * (ny + 1), hx = (nx + 1) / 2;
-        const long len[9] = {nx + 1, nx + 1, nb, nb, nb, nb, nz + 1, nz + 1, nz + 1};
-        for (int i = 0; i < 9; ++i) {
+        const long len[12] = {nx + 1, nx + 1, nb, nb, nb, nb, nz + 1, nz + 1, nz + 1, nz + 1, nz + 1, nz + 1};
+        for (int i = 0; i < 12; ++i) {
             pco[i] = (long)pc.size();
             pc.resize(pc.size() + len[i], 0.0);
         }
-        pco[9] = (long)pc.size();
+        pco[12] = (long)pc.size();
         pc.resize(pc.size() + 2 * hx * ny * nz, 0.0);
         double *ajp1 = &pc[pco[0]], *ajm1 = &pc[pco[1]], *bkp1 = &pc[pco[2]], *bkm1 = &pc[pco[3]];
         double *a2 = &pc[pco[4]], *e2 = &pc[pco[5]], *zpm = &pc[pco[6]], *zpc = &pc[pco[7]], *zcm = &pc[pco[8]];
@@ -552,6 +557,7 @@ int cumc3d_init(const cumc3d_desc *desc, cumc3d_ctx **out) {
             zpm[k] = zp1 - zm1;
             zpc[k] = zp1 - zc;
             zcm[k] = zc - zm1;
+            for (int i = 0; i < 3; ++i) pc[pco[9 + i] + k] = 1.0 / pc[pco[6 + i] + k];
         }
     }
     int rc = 0;
@@ -667,8 +673,8 @@ int cumc3d_init(const cumc3d_desc *desc, cumc3d_ctx **out) {
         }
         x->ajp1 = c0 + pco[0]; x->ajm1 = c0 + pco[1]; x->bkp1 = c0 + pco[2]; x->bkm1 = c0 + pco[3];
         x->sor_a2 = c0 + pco[4]; x->sor_e2 = c0 + pco[5];
-        for (int i = 0; i < 3; ++i) x->sor_z[i] = c0 + pco[6 + i];
-        x->sor_rho = c0 + pco[9];
+        for (int i = 0; i < 6; ++i) x->sor_z[i] = c0 + pco[6 + i];
+        x->sor_rho = c0 + pco[12];
         x->part_max = c0 + pc.size();
         x->part_nan = (long long *)(x->part_max + x->sor_nblk);
     }

@@ -41,8 +41,8 @@
 
 namespace cumc3d {
 
-// colour-split slots of each colour per black block (1024 cells, 4 per thread)
-constexpr int SOR_SLOTS = 512;
+// colour-split slots of each colour per plane of a block, one per thread
+constexpr int SOR_SLOTS = 256;
 
 // Per-cell SOR data are split by colour so that each sweep reads its cells
 // densely: colour c (0 red, 1 black) holds, for row (k, l), the cells
@@ -69,10 +69,11 @@ struct SorArgs {
     const double *ajp1, *ajm1;          // [j], j = 1..nx
     const double *bkp1, *bkm1;          // [k(nx+1) + j]
     const double *a2, *e2;              // [k(nx+1) + j]: 2/xc^2/sin^2 and epsc's radial + polar terms
-    const double *zpm, *zpc, *zcm;      // [l]: zp1-zm1, zp1-zc, zc-zm1
-    long long *part_nan;                // per black block: q of its last NaN term, -1 if none
-    double *part_max;                   // per black block: max of the terms after it, -1 if none
-    int nblk;                           // black blocks: ceil(hx ny / SOR_SLOTS) per plane, times nz
+    const double *z[3], *iz[3];         // [l]: zp1-zm1, zp1-zc, zc-zm1 and their rounded reciprocals
+    long long *part_nan;                // per run of SOR_SLOTS slots of a plane: q of its last NaN term, -1 if none
+    double *part_max;                   // per run: max of the terms after it, -1 if none
+    int runs, items;                    // runs per plane; runs times plane pairs (the blocks' work)
+    int nblk;                           // runs: ceil(hx ny / SOR_SLOTS) per plane, times nz
     int relax_max;
     int zero_ghosts;                    // the first pair after the zero guess: boundary values 0
     int combine;                        // red kernel: block 0 first decides the previous pair's exit
@@ -157,6 +158,7 @@ __global__ void k_grav_start(DevScalars *S, double m_bh, double c_code, double x
 // never read).  An inactive run (finished or stopped) skips the solve.
 __global__ void k_sor_begin(DevScalars *S) {
     S->sor_n = 0;
+    S->sor_nan = 0;
     if (!S->active) {
         S->sor_state = 1;
         S->sor_iter = 0;
@@ -180,39 +182,73 @@ __device__ __forceinline__ long sor_i(const SorArgs &a, int j, int k, int l) {
     return (long)((j - 1) >> 1) + hx * ((long)(k - 1) + (long)a.ny * (l - 1));
 }
 
-// The neighbour values one cell's update reads (custom.f90:548-550): cells
-// of the other colour from `other` (the black start values for a red cell,
-// the new red values for a black one), the boundary values from the start
-// values of the pair: phi(0) = phi(1) and the theta ends copy the cell
-// itself (`own`, its start value), phi(nx+1) = -1, periodic in phi.
-__device__ __forceinline__ void sor_neigh(const SorArgs &a, const double *other, int j, int k, int l, double own,
+// The neighbour values the update of a cell of colour C reads
+// (custom.f90:548-550), for the cell at split index c = sor_i(j, k, l) in a
+// plane l that the block shares: cells of the other colour from `other` (the
+// black start values for a red cell, the new red values for a black one), the
+// boundary values from the start values of the pair: phi(0) = phi(1) and the
+// theta ends copy the cell itself (`own`, its start value), phi(nx+1) = -1,
+// periodic in phi.  In the split order the neighbours sit at fixed offsets:
+// along x at c or c +- 1 by j's parity, along theta at c +- hx, along phi at
+// c +- hx ny.  Every load is unconditional, from a clamped index.
+template <int C>
+__device__ __forceinline__ void sor_neigh(const SorArgs &a, const double *other, int j, int k, int l, int c, double own,
                                           double nb[6]) {
     const bool z0 = a.zero_ghosts;
-    nb[0] = j < a.nx ? other[sor_i(a, j + 1, k, l)] : (z0 ? 0.0 : -1.0);
-    nb[1] = j > 1 ? other[sor_i(a, j - 1, k, l)] : (z0 ? 0.0 : own);
-    nb[2] = k < a.ny ? other[sor_i(a, j, k + 1, l)] : (z0 ? 0.0 : own);
-    nb[3] = k > 1 ? other[sor_i(a, j, k - 1, l)] : (z0 ? 0.0 : own);
-    if (l < a.nz) nb[4] = other[sor_i(a, j, k, l + 1)];
-    else if (z0) nb[4] = 0.0;
-    else nb[4] = (((j + k + 1) & 1) ? a.bin : a.rin)[sor_i(a, j, k, 1)];
-    if (l > 1) nb[5] = other[sor_i(a, j, k, l - 1)];
-    else if (z0) nb[5] = 0.0;
-    else nb[5] = (((j + k + a.nz) & 1) ? a.bin : a.rin)[sor_i(a, j, k, a.nz)];
+    const int hx = (a.nx + 1) >> 1, nh = hx * a.ny, odd = j & 1, wrap = nh * (a.nz - 1);
+    // j + k + l = C modulo 2, so the cell across the periodic boundary has
+    // the colour C + 1 - l, or C + nz - l
+    const double *up = l < a.nz ? other + nh : (((C + 1 - l) & 1) ? a.bin : a.rin) - wrap;
+    const double *dn = l > 1 ? other - nh : (((C + a.nz - l) & 1) ? a.bin : a.rin) + wrap;
+    const double xp = other[j < a.nx ? c + 1 - odd : c], xm = other[j > 1 ? c - odd : c];
+    const double yp = other[k < a.ny ? c + hx : c], ym = other[k > 1 ? c - hx : c];
+    const double zp = up[c], zm = dn[c];
+    nb[0] = j < a.nx ? xp : (z0 ? 0.0 : -1.0);
+    nb[1] = j > 1 ? xm : (z0 ? 0.0 : own);
+    nb[2] = k < a.ny ? yp : (z0 ? 0.0 : own);
+    nb[3] = k > 1 ? ym : (z0 ? 0.0 : own);
+    nb[4] = l == a.nz && z0 ? 0.0 : zp;
+    nb[5] = l == 1 && z0 ? 0.0 : zm;
 }
 
-// one cell's relaxation (custom.f90:544-551); returns the new value
-__device__ __forceinline__ double sor_cell(const SorArgs &a, int j, int k, int l, double rho_in, const double nb[6],
-                                           double old) {
+// The coefficients of a (j, k) column that do not depend on the plane
+struct SorColumn {
+    double A, e2, ajp1, ajm1, bkp1, bkm1;
+};
+__device__ __forceinline__ SorColumn sor_column(const SorArgs &a, int j, int k) {
     const int jk = k * (a.nx + 1) + j;
-    const double A = a.a2[jk], zpc = a.zpc[l], zcm = a.zcm[l];
-    const double t = A / a.zpm[l];
-    const double clp1 = t / zpc, clm1 = t / zcm;
-    const double epsc = a.e2[jk] - A / zpc / zcm;
-    const double s = a.ajp1[j] * nb[0] + a.ajm1[j] * nb[1] + a.bkp1[jk] * nb[2] + a.bkm1[jk] * nb[3] +
-                     clp1 * nb[4] + clm1 * nb[5];
-    const double rhs = (a.pi4 * rho_in - s) / epsc;
+    return {a.a2[jk], a.e2[jk], a.ajp1[j], a.ajm1[j], a.bkp1[jk], a.bkm1[jk]};
+}
+
+// one cell's relaxation (custom.f90:544-551); returns the new value.  The five
+// quotients by the plane's phi spacings take their reciprocals from the table.
+__device__ __forceinline__ double sor_cell(const SorArgs &a, const SorColumn &q, int l, double rho_in,
+                                           const double nb[6], double old) {
+    const Den<double> dpm(a.z[0][l], a.iz[0][l]), dpc(a.z[1][l], a.iz[1][l]), dcm(a.z[2][l], a.iz[2][l]);
+    const double t = dpm(q.A);
+    const double clp1 = dpc(t), clm1 = dcm(t);
+    const double epsc = q.e2 - dcm(dpc(q.A));
+    const double s = q.ajp1 * nb[0] + q.ajm1 * nb[1] + q.bkp1 * nb[2] + q.bkm1 * nb[3] + clp1 * nb[4] + clm1 * nb[5];
+    const double rhs = Den<double>(epsc).tiny(a.pi4 * rho_in - s);
     return (1.0 - a.omega) * old + a.omega * rhs;
 }
+
+// The run and the first plane of a block.  Block row y covers plane l and plane
+// l + 2, whose cells of one colour share (j, k) and with it the column's six
+// coefficients and the plane between them.  Blocks are dealt to the 8 XCDs
+// round-robin; each XCD takes one contiguous eighth of the (row, run) items,
+// the same in both kernels, so that most of what it reads is what it wrote.
+// False for a padding block.
+__device__ __forceinline__ bool sor_item(const SorArgs &a, int block, int &run, int &l0) {
+    const int per = (a.items + 7) >> 3, w = (block & 7) * per + (block >> 3);
+    const int y = w / a.runs;
+    run = w - y * a.runs;
+    l0 = 4 * (y >> 1) + 1 + (y & 1);
+    return (block >> 3) < per && w < a.items && l0 <= a.nz;
+}
+
+// Holds v where it is: a value loaded before a branch is not sunk behind it.
+__device__ __forceinline__ void pin(double &v) { __asm__ volatile("" : "+v"(v)); }
 
 // position of cell i of row (k, l) of a colour in the colour-split rho_in
 __device__ __forceinline__ long sor_rec(const SorArgs &a, int colour, int i, int k, int l) {
@@ -266,6 +302,24 @@ __device__ __forceinline__ double block_max_d(double v) {
     return m;
 }
 
+// Maximum over the wave, in lane 63 (values >= -1, no NaN): DPP moves within
+// rows of 16, then the row broadcasts.
+template <int CTRL> __device__ __forceinline__ double dpp_max(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp((int)b, (int)b, CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp((int)(b >> 32), (int)(b >> 32), CTRL, 0xf, 0xf, false);
+    const double o = __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+    return o > v ? o : v;
+}
+__device__ __forceinline__ double wave_max_d(double v) {
+    v = dpp_max<0x111>(v);   // row_shr:1
+    v = dpp_max<0x112>(v);   // row_shr:2
+    v = dpp_max<0x114>(v);   // row_shr:4
+    v = dpp_max<0x118>(v);   // row_shr:8
+    v = dpp_max<0x142>(v);   // row_bcast:15
+    return dpp_max<0x143>(v);   // row_bcast:31
+}
+
 // Two partials of consecutive q ranges, the right one folded into the left:
 // the last NaN of the right range supersedes everything before it.
 __device__ __forceinline__ void fold_partial(long long &L, double &M, long long L2, double M2) {
@@ -278,33 +332,56 @@ __device__ __forceinline__ void fold_partial(long long &L, double &M, long long 
 }
 
 // The previous pair's abserror from the black blocks' partials and the exit
-// decision (custom.f90:638, :644), by one block of 256 threads.  The
-// partials are in q order (block index plane-major), so their left-to-right
-// fold is (the last NaN q, the maximum of the terms after it): each thread
-// folds a contiguous run of them, then the threads' results are folded in
-// thread order (lane i takes lane i + off at each level of the tree).
+// decision (custom.f90:638, :644), by one block of 256 threads.  Most pairs
+// have no NaN term (a block that has one sets sor_nan): then abserror is the
+// maximum of the runs' maxima in any order, and each thread takes every 256th
+// run, its loads in flight together.
+// Else the partials are folded left to right (they are in q order: the last
+// NaN q, and the maximum of the terms after it): each thread folds a
+// contiguous run of them, then the threads' results are folded in thread
+// order (lane i takes lane i + off at each level of the tree).
 __device__ void sor_decide(const SorArgs &a) {
     DevScalars *S = a.S;
-    const int per = (a.nblk + 255) >> 8;
-    const int i0 = (int)threadIdx.x * per, i1 = i0 + per < a.nblk ? i0 + per : a.nblk;
-    long long L = -1;
-    double M = -1.0;
-    for (int i = i0; i < i1; ++i) fold_partial(L, M, a.part_nan[i], a.part_max[i]);
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const long long L2 = __shfl_down(L, off, 64);
-        const double M2 = __shfl_down(M, off, 64);
-        if ((threadIdx.x & 63) + off < 64) fold_partial(L, M, L2, M2);
-    }
-    __shared__ long long wl[4];
     __shared__ double wm[4];
-    if ((threadIdx.x & 63) == 0) {
-        wl[threadIdx.x >> 6] = L;
-        wm[threadIdx.x >> 6] = M;
+    __shared__ long long wl[4];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nan = S->sor_nan;
+    double M = -1.0;
+    for (int i0 = threadIdx.x; i0 < a.nblk; i0 += 16 * 256) {
+        double v[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v[u] = i0 + 256 * u < a.nblk ? a.part_max[i0 + 256 * u] : -1.0;
+#pragma unroll
+        for (int u = 0; u < 16; ++u) M = v[u] > M ? v[u] : M;
+    }
+    long long L = -1;
+    if (nan) {
+        const int per = (a.nblk + 255) >> 8;
+        const int i0 = (int)threadIdx.x * per, i1 = i0 + per < a.nblk ? i0 + per : a.nblk;
+        M = -1.0;
+        for (int i = i0; i < i1; ++i) fold_partial(L, M, a.part_nan[i], a.part_max[i]);
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const long long L2 = __shfl_down(L, off, 64);
+            const double M2 = __shfl_down(M, off, 64);
+            if (lane + off < 64) fold_partial(L, M, L2, M2);
+        }
+        if (lane == 0) {
+            wl[wv] = L;
+            wm[wv] = M;
+        }
+    } else {
+        M = wave_max_d(M);
+        if (lane == 63) {
+            wl[wv] = -1;
+            wm[wv] = M;
+        }
     }
     __syncthreads();
     if (threadIdx.x != 0) return;
-    for (int w = 1; w < (int)(blockDim.x >> 6); ++w) fold_partial(L, M, wl[w], wm[w]);
+    L = wl[0];
+    M = wm[0];
+    for (int w = 1; w < 4; ++w) fold_partial(L, M, wl[w], wm[w]);
+    S->sor_nan = 0;
     const long long N = (long long)a.nx * a.ny * a.nz;
     double err;
     if (L == N - 1) err = 1.0e-50;   // the private result is NaN: the combine keeps 1e-50
@@ -321,85 +398,148 @@ __device__ void sor_decide(const SorArgs &a) {
     }
 }
 
-// Red cells ((j + k + l) even), every second cell along x: grid (x: the
-// plane's red cells / 256 + 1 for the decision block, y: l - 1).  With
-// `combine`, block (0, 0) first decides the previous pair's exit; the other
-// blocks do not wait for it: a pair begun after the solve ended only writes
-// the buffer that is not the result, and the black kernel and every later
-// kernel see the decision and return.
+// Red cells ((j + k + l) even).  With `combine`, block 0 decides the previous
+// pair's exit (the work items start at block 8); the others do not wait for it:
+// a pair begun after the solve ended only writes the buffer that is not the
+// result, and the black kernel and every later kernel see the decision and
+// return.  At the sizes of a progenitor grid (156 x 44 x 128) the arrays sit in
+// the Infinity Cache and both kernels are bound by its latency and the launch
+// (fewer instructions no longer help): each thread takes two cells that share
+// their column, loads everything before it looks at the end flag, divides by
+// reciprocals, and finds its planes on the XCD that wrote them.  A solve of
+// 10496 pairs took 196 ms (18.7 us a pair); two planes a thread with
+// reciprocals 172, fixed neighbour offsets and the order-free fold 164, the
+// XCD order 157 ms (15.0 us).
 __global__ __launch_bounds__(256) void k_sor_red(SorArgs a) {
-    if (a.combine && blockIdx.x == 0 && blockIdx.y == 0) {
-        if (!a.S->sor_state && a.S->active) sor_decide(a);
+    if (blockIdx.x < 8) {
+        if (a.combine && blockIdx.x == 0 && !a.S->sor_state && a.S->active) sor_decide(a);
         return;
     }
-    if (a.S->sor_state || !a.S->active) return;
-    const int hx = (a.nx + 1) >> 1;
-    const unsigned t = (blockIdx.x - 1) * blockDim.x + threadIdx.x;
-    if (t >= (unsigned)(hx * a.ny)) return;
-    const int k = 1 + (int)(t / (unsigned)hx), i = (int)(t - (unsigned)(k - 1) * hx), l = 1 + blockIdx.y;
-    const int j = (((1 + k + l) & 1) == 0 ? 1 : 2) + 2 * i;
+    const bool stop = a.S->sor_state || !a.S->active;
+    const int hx = (a.nx + 1) >> 1, nh = hx * a.ny;
+    int run, l0;
+    if (!sor_item(a, blockIdx.x - 8, run, l0)) return;
+    const int s = run * SOR_SLOTS + (int)threadIdx.x;
+    if (s >= nh) return;
+    const int k = 1 + s / hx, i = s - (k - 1) * hx;
+    const int j = (((1 + k + l0) & 1) == 0 ? 1 : 2) + 2 * i;
     if (j > a.nx) return;
-    const long ic = sor_i(a, j, k, l);
-    const double rho_in = a.rho_in[sor_rec(a, 0, i, k, l)];
-    const double old = a.rin[ic];
-    double nb[6];
-    sor_neigh(a, a.bin, j, k, l, old, nb);
-    a.rout[ic] = sor_cell(a, j, k, l, rho_in, nb, old);
+    const bool two = l0 + 2 <= a.nz;
+    const SorColumn q = sor_column(a, j, k);
+    double rho_in[2], old[2], nb[2][6];
+    int ic[2];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        const int l = p && two ? l0 + 2 : l0;
+        ic[p] = s + nh * (l - 1);   // sor_i(a, j, k, l)
+        rho_in[p] = a.rho_in[ic[p]];
+        old[p] = a.rin[ic[p]];
+        sor_neigh<0>(a, a.bin, j, k, l, ic[p], old[p], nb[p]);
+    }
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        pin(rho_in[p]);
+        for (int v = 0; v < 6; ++v) pin(nb[p][v]);
+    }
+    if (stop) return;
+    const double n0 = sor_cell(a, q, l0, rho_in[0], nb[0], old[0]);
+    a.rout[ic[0]] = n0;
+    if (two) a.rout[ic[1]] = sor_cell(a, q, l0 + 2, rho_in[1], nb[1], old[1]);
 }
 
-// Every interior cell, in the colour-split order: block b of plane l takes
-// the split indices [b S, (b+1) S) of both colours (S = SOR_SLOTS), the cells
-// (k, j = 2i+1, 2i+2) of rows k at index i; together they are one contiguous
-// range of q.  A thread's slots 0-1 are black cells, which relax from the new
-// red values, and its slots 2-3 red ones, so the lanes of a wave share a
-// colour and neither branch diverges.  Every cell forms its error term
-// |dphi/phi_old| (custom.f90:593) from the pair's start and end values, and
-// the block folds them into its partial: the fold is a maximum, so the order
-// of the slots does not matter.
+// Every interior cell, in the colour-split order: a block takes one run of
+// SOR_SLOTS split indices of both colours in each of its two planes; in a plane
+// those are the cells (k, j = 2i+1, 2i+2), one contiguous range of q.  A thread
+// relaxes the black cell of its slot from the new red values and forms the
+// error terms |dphi/phi_old| (custom.f90:593) of its black and red cell from
+// the pair's start and end values; the run's partial is their fold.  Without a
+// NaN in the block (its waves vote) that is one maximum per plane.
 __global__ __launch_bounds__(256) void k_sor_black(SorArgs a) {
-    if (a.S->sor_state || !a.S->active) return;
+    const bool stop = a.S->sor_state || !a.S->active;
     const int hx = (a.nx + 1) >> 1, nh = hx * a.ny, nxy = a.nx * a.ny;
-    const int l = 1 + blockIdx.y;
-    double e[4];
-    long long qq[4];
-    long long last = -1;
+    int run, l0;
+    if (!sor_item(a, blockIdx.x, run, l0)) return;
+    const bool two = l0 + 2 <= a.nz;
+    const int s = run * SOR_SLOTS + (int)threadIdx.x;
+    const int sc = s < nh ? s : nh - 1;
+    const int k = 1 + sc / hx, i = sc - (k - 1) * hx;
+    const int jb = (((1 + k + l0) & 1) == 1 ? 1 : 2) + 2 * i, jr = (((1 + k + l0) & 1) == 0 ? 1 : 2) + 2 * i;
+    // the padded slot of an odd row holds no cell; its thread reads the row's last one
+    const bool lb = s < nh && jb <= a.nx, lr = s < nh && jr <= a.nx;
+    const int j = jb <= a.nx ? jb : a.nx;
+    const SorColumn q = sor_column(a, j, k);
+    double rho_in[2], bold[2], rold[2], rnew[2], nb[2][6];
+    int ic[2];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        const int colour = u < 2 ? 1 : 0;
-        const int s = blockIdx.x * SOR_SLOTS + (u & 1) * 256 + (int)threadIdx.x;
-        qq[u] = -1;
-        e[u] = -1.0;
-        if (s >= nh) continue;
-        const int k = 1 + s / hx, i = s - (k - 1) * hx;
-        const int j = (((1 + k + l) & 1) == colour ? 1 : 2) + 2 * i;
-        if (j > a.nx) continue;   // the padded slot of an odd row
-        qq[u] = (long long)(l - 1) * nxy + (long long)(k - 1) * a.nx + (j - 1);
-        const long ic = (long)s + (long)nh * (l - 1);   // sor_i(a, j, k, l)
-        double old, nw;
-        if (colour) {
-            const double rho_in = a.rho_in[(long)nh * a.nz + ic];   // sor_rec(a, 1, i, k, l)
-            old = a.bin[ic];
-            double nb[6];
-            sor_neigh(a, a.rout, j, k, l, old, nb);
-            nw = sor_cell(a, j, k, l, rho_in, nb, old);
-            a.bout[ic] = nw;
-        } else {
-            old = a.rin[ic];
-            nw = a.rout[ic];
-        }
-        e[u] = fabs((nw - old) / old);
-        if (e[u] != e[u]) last = qq[u] > last ? qq[u] : last;
+    for (int p = 0; p < 2; ++p) {
+        const int l = p && two ? l0 + 2 : l0;
+        ic[p] = sc + nh * (l - 1);   // sor_i of both cells
+        rho_in[p] = (a.rho_in + nh * a.nz)[ic[p]];
+        bold[p] = a.bin[ic[p]];
+        rold[p] = a.rin[ic[p]];
+        rnew[p] = a.rout[ic[p]];
+        sor_neigh<1>(a, a.rout, j, k, l, ic[p], bold[p], nb[p]);
     }
-    last = block_max_ll(last);
-    double m = -1.0;
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
-        if (qq[u] > last && e[u] == e[u]) m = e[u] > m ? e[u] : m;
-    m = block_max_d(m);
-    if (threadIdx.x == 0) {
-        const int b = blockIdx.y * gridDim.x + blockIdx.x;
-        a.part_nan[b] = last;
-        a.part_max[b] = m;
+    for (int p = 0; p < 2; ++p) {
+        pin(rho_in[p]);
+        pin(rold[p]);
+        pin(rnew[p]);
+        for (int v = 0; v < 6; ++v) pin(nb[p][v]);
+    }
+    if (stop) return;
+    double eb[2], er[2];
+    bool bad = false;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        const bool on = p == 0 || two;
+        eb[p] = er[p] = -1.0;
+        if (lb && on) {
+            const double nw = sor_cell(a, q, p ? l0 + 2 : l0, rho_in[p], nb[p], bold[p]);
+            a.bout[ic[p]] = nw;
+            eb[p] = fabs((nw - bold[p]) / bold[p]);
+        }
+        if (lr && on) er[p] = fabs((rnew[p] - rold[p]) / rold[p]);
+        bad = bad || eb[p] != eb[p] || er[p] != er[p];
+    }
+    __shared__ double wm[2][4];
+    __shared__ int wbad[4];
+    const int w = threadIdx.x >> 6;
+    const int vote = __ballot(bad) != 0;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        const double m = wave_max_d(eb[p] > er[p] ? eb[p] : er[p]);
+        if ((threadIdx.x & 63) == 63) wm[p][w] = m;
+    }
+    if ((threadIdx.x & 63) == 63) wbad[w] = vote;
+    __syncthreads();
+    const bool any = wbad[0] | wbad[1] | wbad[2] | wbad[3];
+    const int b = (l0 - 1) * a.runs + run;
+    if (!any) {
+        if (threadIdx.x < (two ? 2 : 1)) {
+            const double *v = wm[threadIdx.x];
+            double m = v[0];
+            for (int u = 1; u < 4; ++u) m = v[u] > m ? v[u] : m;
+            a.part_nan[b + threadIdx.x * 2 * a.runs] = -1;
+            a.part_max[b + threadIdx.x * 2 * a.runs] = m;
+        }
+        return;
+    }
+    for (int p = 0; p < (two ? 2 : 1); ++p) {
+        const long long q0 = (long long)(l0 + 2 * p - 1) * nxy + (long long)(k - 1) * a.nx - 1;
+        long long last = -1;
+        if (er[p] != er[p]) last = q0 + jr;
+        if (eb[p] != eb[p]) last = q0 + jb > last ? q0 + jb : last;
+        last = block_max_ll(last);
+        double m = -1.0;
+        if (q0 + jb > last && eb[p] == eb[p]) m = eb[p];
+        if (q0 + jr > last && er[p] == er[p]) m = er[p] > m ? er[p] : m;
+        m = block_max_d(m);
+        if (threadIdx.x == 0) {
+            a.part_nan[b + 2 * p * a.runs] = last;
+            a.part_max[b + 2 * p * a.runs] = m;
+            a.S->sor_nan = 1;
+        }
     }
 }
 

@@ -39,7 +39,7 @@ struct DevScalars {
     int sor_n;                        // sweeps done in the running solve
     int sor_iter;                     // the DO variable n when the solve ended
     int grav_stop;                    // 1: r_sh reached xF(0) (the reference STOPs)
-    int pad2;
+    int sor_nan;                      // the last sweep pair had a NaN error term
 };
 
 struct Axis {

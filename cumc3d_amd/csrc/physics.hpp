@@ -76,6 +76,8 @@ template <> struct Den<double> {
         const double e = __builtin_fma(-x, y, 1.0);
         y = __builtin_fma(__builtin_fma(e, e, e), y, y);
     }
+    // a denominator with its correctly rounded reciprocal
+    __device__ __forceinline__ Den(double x, double inv) : d(x), y(inv) {}
     __device__ __forceinline__ double operator()(double n) const {
         const double q = n * y;
         return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-d, q, n), y, q), d, n);
