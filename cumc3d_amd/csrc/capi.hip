@@ -100,7 +100,7 @@ __global__ void k_dt_finalize(DevScalars *S) {
     double dt = fmin2(1.0e5, m);
     if (S->t + dt > S->total_time) dt = S->total_time - S->t;
     S->dt = dt;
-    S->dtmin_bits = (unsigned long long)__double_as_longlong(1.0e300);
+    S->dtmin_bits = DTMIN_NONE;
 }
 
 __global__ void k_time_advance(DevScalars *S, double *dtlog, int slot) {
@@ -111,13 +111,29 @@ __global__ void k_time_advance(DevScalars *S, double *dtlog, int slot) {
     if (dtlog) dtlog[slot] = S->dt;
 }
 
-__global__ void k_set_dt(DevScalars *S, double dt) {
+// The step's dt from the host; `reset`: the minimum has been taken (cumc3d_finddt)
+__global__ void k_set_dt(DevScalars *S, double dt, int reset) {
     S->dt = dt;
     S->active = !S->grav_stop;
+    if (reset) {
+        S->dtmin_bits = DTMIN_NONE;
+        S->nonfinite = 0;
+    }
 }
 
-// a new initial model starts a run afresh: no model STOP pending
-__global__ void k_clear_stop(DevScalars *S) { S->grav_stop = 0; }
+// a new initial model starts a run afresh: no model STOP pending, the stage kernels active
+__global__ void k_restart(DevScalars *S) {
+    S->grav_stop = 0;
+    S->dt = 0.0;
+    S->active = 1;
+}
+
+__global__ void k_reset_dtmin(DevScalars *S) {
+    S->dtmin_bits = DTMIN_NONE;
+    S->nonfinite = 0;
+}
+
+__global__ void k_publish(const DevScalars *S, HostScalars *pub) { publish(S, pub); }
 
 // SPATIAL on its own runs the stage kernels whatever the run's end time
 __global__ void k_activate(DevScalars *S) { S->active = !S->grav_stop; }
@@ -337,11 +353,32 @@ static int grav_check(cumc3d_ctx *x) {
     return 0;
 }
 
-static int run_stage(cumc3d_ctx *x, int stage) {
+// `pub`: where the ghost fill leaves the CFL minimum for the host, or null
+static int run_stage(cumc3d_ctx *x, int stage, HostScalars *pub) {
     if (stage == 1) sel_refresh(x);
-    if (x->fp32) f32::run_stage(x, stage);
-    else run_stage_t<double>(x, stage);
+    if (x->fp32) f32::run_stage(x, stage, pub);
+    else run_stage_t<double>(x, stage, pub);
     return grav_stage(x, stage);
+}
+
+// The device minimum starts over before the next reduction, if cumc3d_finddt
+// has taken it.
+static void settle_dtmin(cumc3d_ctx *x) {
+    if (x->dt_taken) hipLaunchKernelGGL(k_reset_dtmin, dim3(1), dim3(1), 0, x->stream, x->S);
+    x->dt_taken = false;
+}
+
+// Device memory of at least n doubles (n <= 9 G) between steps.  The sweeps
+// write every flux before it is read, so the flux arrays serve, except with
+// HLL, whose faces without a branch keep the flux of an earlier sweep.
+static int staging(cumc3d_ctx *x, size_t n, DevTmp &own, double **p) {
+    if (x->d.riemann != CUMC3D_HLL) {
+        *p = (double *)x->F[0][0];
+        return 0;
+    }
+    HIPCHK(hipMalloc(&own.p, n * sizeof(double)));
+    *p = (double *)own.p;
+    return 0;
 }
 
 // per-kernel-class device times from the recorded events (after a sync)
@@ -567,26 +604,40 @@ int cumc3d_init(const cumc3d_desc *desc, cumc3d_ctx **out) {
         return fail(CUMC3D_EHIP, "hipStreamCreate failed");
     }
     if (int e = scratch_address(&x->scratch)) { cleanup(); return e; }
-    if (hipMalloc(&x->met, hm.size() * sizeof(double)) != hipSuccess) { cleanup(); return fail(CUMC3D_ENOMEM, "metrics"); }
-    if (hipMemcpy(x->met, hm.data(), hm.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess) {
+    // one allocation: metrics, weights in the working type, HLLD carry slots
+    x->fp32 = d.precision == CUMC3D_FP32;
+    const size_t wsz = x->fp32 ? sizeof(float) : sizeof(double);
+    if (const char *mt = getenv("CUMC3D_MARCH_THREADS")) {
+        long v = atol(mt);
+        if (v >= 1) x->march_threads = v;
+    }
+    size_t slots[4] = {};
+    if (d.riemann == CUMC3D_HLLD && d.hlld_bn_mode == 2)
+        for (int D = 0; D < 3; ++D) {
+            int ns;
+            const dim3 g = sweep_grid(x, D, ns);
+            slots[D + 1] = slots[D] + (D < d.n_dim ? (size_t)g.x * g.y : 0);
+        }
+    const size_t wat = (hm.size() * sizeof(double) + 255) / 256 * 256;
+    const size_t sat = wat + (hw.size() * wsz + 255) / 256 * 256;
+    std::vector<char> block(sat);
+    memcpy(block.data(), hm.data(), hm.size() * sizeof(double));
+    for (size_t i = 0; i < hw.size(); ++i) {
+        if (x->fp32) ((float *)(block.data() + wat))[i] = (float)hw[i];
+        else ((double *)(block.data() + wat))[i] = hw[i];
+    }
+    if (hipMalloc(&x->met, sat + slots[3] * sizeof(double2)) != hipSuccess) { cleanup(); return fail(CUMC3D_ENOMEM, "metrics"); }
+    if (hipMemcpy(x->met, block.data(), sat, hipMemcpyHostToDevice) != hipSuccess) {
         cleanup();
         return fail(CUMC3D_EHIP, "metric upload");
     }
-    x->fp32 = d.precision == CUMC3D_FP32;
-    const size_t wsz = x->fp32 ? sizeof(float) : sizeof(double);
-    std::vector<float> hw32;
-    if (x->fp32) hw32.assign(hw.begin(), hw.end());
-    if (hipMalloc(&x->wtab, hw.size() * wsz) != hipSuccess) { cleanup(); return fail(CUMC3D_ENOMEM, "weights"); }
-    if (hipMemcpy(x->wtab, x->fp32 ? (const void *)hw32.data() : hw.data(), hw.size() * wsz, hipMemcpyHostToDevice) !=
-        hipSuccess) {
-        cleanup();
-        return fail(CUMC3D_EHIP, "weight upload");
-    }
+    if (slots[3])
+        for (int D = 0; D < 3; ++D) x->slot[D] = (double2 *)((char *)x->met + sat) + slots[D];
     for (int a = 0; a < 3; ++a) {
         x->ax[a].xF = x->met + off[a][0];
         x->ax[a].d = x->met + off[a][1];
         x->ax[a].c = x->met + off[a][2];
-        const auto table = [&](int i) { return (const char *)x->wtab + off[a][i] * wsz; };
+        const auto table = [&](int i) { return (const char *)x->met + wat + off[a][i] * wsz; };
         x->ax[a].w = table(3);
         for (int sch = 0; sch < 3; ++sch) x->ax[a].wsel[sch] = table(4 + sch);
     }
@@ -627,22 +678,12 @@ int cumc3d_init(const cumc3d_desc *desc, cumc3d_ctx **out) {
     memset(&s0, 0, sizeof(s0));
     s0.total_time = 1.0e300;
     s0.active = 1;
-    s0.dtmin_bits = (unsigned long long)0x7E37E43C8800759CULL;   // bits of 1e300
+    s0.dtmin_bits = DTMIN_NONE;
     s0.m_bh = s0.mbh_old = x->grav_p.m_bh;
     if (hipMemcpy(x->S, &s0, sizeof(s0), hipMemcpyHostToDevice) != hipSuccess) { cleanup(); return fail(CUMC3D_EHIP, "scalars"); }
-    if (const char *mt = getenv("CUMC3D_MARCH_THREADS")) {
-        long v = atol(mt);
-        if (v >= 1) x->march_threads = v;
-    }
-    if (d.riemann == CUMC3D_HLLD && d.hlld_bn_mode == 2) {
-        size_t at[4] = {};
-        for (int D = 0; D < 3; ++D) {
-            int ns;
-            const dim3 g = sweep_grid(x, D, ns);
-            at[D + 1] = at[D] + (D < d.n_dim ? (size_t)g.x * g.y : 0);
-        }
-        if (hipMalloc(&x->slot[0], at[3] * sizeof(double2)) != hipSuccess) { cleanup(); return fail(CUMC3D_ENOMEM, "carry slots"); }
-        for (int D = 1; D < 3; ++D) x->slot[D] = x->slot[0] + at[D];
+    if (hipHostMalloc((void **)&x->pub, sizeof(HostScalars), hipHostMallocDefault) != hipSuccess) {
+        cleanup();
+        return fail(CUMC3D_ENOMEM, "host scalars");
     }
     if (d.riemann == CUMC3D_HLL) {
         if (hipMalloc(&x->stale, (size_t)3 * x->G) != hipSuccess) { cleanup(); return fail(CUMC3D_ENOMEM, "stale flags"); }
@@ -687,8 +728,8 @@ int cumc3d_upload(cumc3d_ctx *x, const double *prim, const double *eps, const do
     if ((x->d.model == CUMC3D_MODEL_TORUS || x->d.model == CUMC3D_MODEL_TORUS_SPH) && !floors3)
         return fail(CUMC3D_EINVAL, "torus models need floor arrays");
     DevTmp buf;
-    HIPCHK(hipMalloc(&buf.p, (size_t)9 * x->G * sizeof(double)));
-    double *tmp = (double *)buf.p;
+    double *tmp;
+    if (int rc = staging(x, (size_t)9 * x->G, buf, &tmp)) return rc;
     HIPCHK(hipMemcpyAsync(tmp, prim, (size_t)8 * x->G * sizeof(double), hipMemcpyHostToDevice, x->stream));
     HIPCHK(hipMemcpyAsync(tmp + (size_t)8 * x->G, eps, x->G * sizeof(double), hipMemcpyHostToDevice, x->stream));
     x->cur = 0;
@@ -710,8 +751,7 @@ int cumc3d_upload(cumc3d_ctx *x, const double *prim, const double *eps, const do
 int cumc3d_initial_update(cumc3d_ctx *x) {
     if (!x) return fail(CUMC3D_EINVAL, "null context");
     if (!x->uploaded) return fail(CUMC3D_ESTATE, "upload an initial model first");
-    hipLaunchKernelGGL(k_clear_stop, dim3(1), dim3(1), 0, x->stream, x->S);
-    hipLaunchKernelGGL(k_set_dt, dim3(1), dim3(1), 0, x->stream, x->S, 0.0);   // also re-activates the stage kernels
+    hipLaunchKernelGGL(k_restart, dim3(1), dim3(1), 0, x->stream, x->S);
     const unsigned gi = nblk((long)x->nx * x->ny * x->nz), gg = nblk(x->G);
     if (x->fp32) {
         f32::initial_update(x);
@@ -739,21 +779,20 @@ int cumc3d_initial_update(cumc3d_ctx *x) {
 int cumc3d_finddt(cumc3d_ctx *x, double *dt) {
     if (!x || !dt) return fail(CUMC3D_EINVAL, "null argument");
     if (!x->initialized) return fail(CUMC3D_ESTATE, "call cumc3d_initial_update first");
-    if (!x->dt_pending) launch_finddt(x);
+    if (!x->dt_pending) {
+        settle_dtmin(x);
+        launch_finddt(x);
+        hipLaunchKernelGGL(k_publish, dim3(1), dim3(1), 0, x->stream, x->S, x->pub);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipStreamSynchronize(x->stream));
+    }
+    // (pending: the step before left the minimum of its result in pub)
     x->dt_pending = false;
-    unsigned long long bits = 0;
-    int bad = 0;
-    HIPCHK(hipMemcpyAsync(&bits, &x->S->dtmin_bits, sizeof(bits), hipMemcpyDeviceToHost, x->stream));
-    HIPCHK(hipMemcpyAsync(&bad, &x->S->nonfinite, sizeof(bad), hipMemcpyDeviceToHost, x->stream));
-    HIPCHK(hipStreamSynchronize(x->stream));
+    x->dt_taken = true;
+    const int bad = x->pub->nonfinite;
     double m;
-    memcpy(&m, &bits, sizeof(m));
+    memcpy(&m, &x->pub->dtmin_bits, sizeof(m));
     *dt = m < 1.0e5 ? m : 1.0e5;
-    unsigned long long reset = 0x7E37E43C8800759CULL;
-    const int clear = 0;
-    HIPCHK(hipMemcpyAsync(&x->S->dtmin_bits, &reset, sizeof(reset), hipMemcpyHostToDevice, x->stream));
-    HIPCHK(hipMemcpyAsync(&x->S->nonfinite, &clear, sizeof(clear), hipMemcpyHostToDevice, x->stream));
-    HIPCHK(hipStreamSynchronize(x->stream));
     if (bad)
         return fail(CUMC3D_ENONFINITE,
                     "a cell's CFL time step was NaN or non-positive (NaN or negative energy in the state)");
@@ -766,10 +805,11 @@ int cumc3d_rk3_step(cumc3d_ctx *x, double dt) {
     if (!x->initialized) return fail(CUMC3D_ESTATE, "call cumc3d_initial_update first");
     if (x->next_stage != 1) return fail(CUMC3D_ESTATE, "a step run by cumc3d_stage is not finished");
     if (int rc = grav_check(x)) return rc;
-    hipLaunchKernelGGL(k_set_dt, dim3(1), dim3(1), 0, x->stream, x->S, dt);
+    hipLaunchKernelGGL(k_set_dt, dim3(1), dim3(1), 0, x->stream, x->S, dt, (int)x->dt_taken);
+    x->dt_taken = false;
     x->cur_step = x->nstep_total;
     for (int s = 1; s <= 3; ++s)
-        if (int rc = run_stage(x, s)) return rc;
+        if (int rc = run_stage(x, s, s == 3 ? x->pub : nullptr)) return rc;
     x->nstep_total += 1;
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(x->stream));
@@ -785,12 +825,13 @@ int cumc3d_stage(cumc3d_ctx *x, int stage, double dt) {
     if (stage < 1 || stage > 3) return fail(CUMC3D_EINVAL, "stage must be 1, 2 or 3");
     if (stage != x->next_stage) return fail(CUMC3D_ESTATE, "the stages of a step run in the order 1, 2, 3");
     if (int rc = grav_check(x)) return rc;
-    hipLaunchKernelGGL(k_set_dt, dim3(1), dim3(1), 0, x->stream, x->S, dt);
+    hipLaunchKernelGGL(k_set_dt, dim3(1), dim3(1), 0, x->stream, x->S, dt, (int)x->dt_taken);
+    x->dt_taken = false;
     if (stage == 1) {
         x->cur_step = x->nstep_total;
         x->dt_pending = false;
     }
-    if (int rc = run_stage(x, stage)) return rc;
+    if (int rc = run_stage(x, stage, stage == 3 ? x->pub : nullptr)) return rc;
     x->next_stage = stage % 3 + 1;
     if (stage == 3) {
         x->nstep_total += 1;
@@ -831,6 +872,11 @@ static int run_loop(cumc3d_ctx *x, int max_steps, double total_time, int sync_ea
     h.t = *t;
     h.total_time = total_time;
     h.nstep = 0;
+    if (x->dt_taken) {
+        h.dtmin_bits = DTMIN_NONE;
+        h.nonfinite = 0;
+        x->dt_taken = false;
+    }
     HIPCHK(hipMemcpy(x->S, &h, sizeof(h), hipMemcpyHostToDevice));
     if (x->timing) {
         if (x->ev.empty()) {
@@ -856,7 +902,7 @@ static int run_loop(cumc3d_ctx *x, int max_steps, double total_time, int sync_ea
         if (!x->dt_pending) launch_finddt(x);
         hipLaunchKernelGGL(k_dt_finalize, dim3(1), dim3(1), 0, x->stream, x->S);
         x->cur_step = x->nstep_total + n;
-        for (int s = 1; s <= 3 && !grc; ++s) grc = run_stage(x, s);
+        for (int s = 1; s <= 3 && !grc; ++s) grc = run_stage(x, s, nullptr);
         x->dt_pending = true;
         hipLaunchKernelGGL(k_time_advance, dim3(1), dim3(1), 0, x->stream, x->S, dlog, n);
         if (sync_each_step) {
@@ -877,6 +923,8 @@ static int run_loop(cumc3d_ctx *x, int max_steps, double total_time, int sync_ea
     HIPCHK(hipStreamSynchronize(x->stream));
     HIPCHK(hipMemcpy(&h, x->S, sizeof(h), hipMemcpyDeviceToHost));
     *t = h.t;
+    x->pub->dtmin_bits = h.dtmin_bits;   // as a step under the host's dt leaves it
+    x->pub->nonfinite = 0;               // reported below
     int done = h.nstep;
     x->nstep_total += done;
     if (steps_done) *steps_done = done;
@@ -899,9 +947,15 @@ int cumc3d_run(cumc3d_ctx *x, int max_steps, double total_time, int sync_each_st
     if (!x || !t) return fail(CUMC3D_EINVAL, "null argument");
     if (!x->initialized) return fail(CUMC3D_ESTATE, "call cumc3d_initial_update first");
     if (x->next_stage != 1) return fail(CUMC3D_ESTATE, "a step run by cumc3d_stage is not finished");
-    DevTmp dbuf;
-    if (dts && max_steps > 0) HIPCHK(hipMalloc(&dbuf.p, (size_t)max_steps * sizeof(double)));
-    return run_loop(x, max_steps, total_time, sync_each_step, t, dts, steps_done, (double *)dbuf.p);
+    if (dts && max_steps > x->dlog_cap) {   // the dt log, kept for the next call
+        if (x->dlog) HIPCHK(hipFree(x->dlog));
+        x->dlog = nullptr;
+        x->dlog_cap = 0;
+        HIPCHK(hipMalloc(&x->dlog, (size_t)max_steps * sizeof(double)));
+        x->dlog_cap = max_steps;
+    }
+    return run_loop(x, max_steps, total_time, sync_each_step, t, dts, steps_done,
+                    dts && max_steps > 0 ? x->dlog : nullptr);
 }
 
 int cumc3d_run_noalloc(cumc3d_ctx *x, int max_steps, double total_time, int sync_each_step, double *t,
@@ -921,9 +975,9 @@ int cumc3d_run_noalloc(cumc3d_ctx *x, int max_steps, double total_time, int sync
 int cumc3d_download(cumc3d_ctx *x, double *prim, double *eps, double *bcell, double *cs) {
     if (!x) return fail(CUMC3D_EINVAL, "null context");
     DevTmp buf;
-    if (prim || bcell) HIPCHK(hipMalloc(&buf.p, (size_t)8 * x->G * sizeof(double)));
-    if (!buf.p && x->fp32 && (eps || cs)) HIPCHK(hipMalloc(&buf.p, (size_t)x->G * sizeof(double)));
-    double *tmp = (double *)buf.p;
+    double *tmp = nullptr;
+    if (prim || bcell || (x->fp32 && (eps || cs)))
+        if (int rc = staging(x, (size_t)(prim || bcell ? 8 : 1) * x->G, buf, &tmp)) return rc;
     const unsigned gg = nblk(x->G);
     if (prim) {
         if (x->fp32) f32::join_prim(x, tmp);
@@ -961,8 +1015,8 @@ int cumc3d_profile(cumc3d_ctx *x, double *primitive, double *epsilon, double *bf
     const size_t np = (size_t)(x->nx + 2) * (x->ny + 2) * (x->nz + 2);
     const size_t nb = (size_t)(x->nx + 3) * (x->ny + 3) * (x->nz + 3);
     DevTmp buf;
-    HIPCHK(hipMalloc(&buf.p, (5 * np + np + 3 * nb) * sizeof(double)));
-    double *tmp = (double *)buf.p;
+    double *tmp;
+    if (int rc = staging(x, 6 * np + 3 * nb, buf, &tmp)) return rc;
     double *dp = primitive ? tmp : nullptr, *de = epsilon ? tmp + 5 * np : nullptr,
            *db = bfield ? tmp + 6 * np : nullptr;
     if (x->fp32)
@@ -1013,10 +1067,10 @@ int cumc3d_finalize(cumc3d_ctx *x) {
     for (auto &e : x->ev) hipEventDestroy(e);
     if (x->pool) hipFree(x->pool);
     if (x->met) hipFree(x->met);
-    if (x->wtab) hipFree(x->wtab);
     if (x->S) hipFree(x->S);
     if (x->stale) hipFree(x->stale);
-    if (x->slot[0]) hipFree(x->slot[0]);
+    if (x->dlog) hipFree(x->dlog);
+    if (x->pub) hipHostFree(x->pub);
     if (x->grav) hipFree(x->grav);
     if (x->ev_x) hipEventDestroy(x->ev_x);
     if (x->ev_m) hipEventDestroy(x->ev_m);

@@ -22,8 +22,7 @@ struct cumc3d_ctx {
     hipStream_t stream = nullptr;
     void *pool = nullptr;         // all per-cell fields
     bool fp32 = false;            // CUMC3D_FP32: working fields are float
-    double *met = nullptr;        // grid metrics
-    void *wtab = nullptr;         // reconstruction weights in the working type
+    double *met = nullptr;        // grid metrics, reconstruction weights, carry slots
     cumc3d::DevScalars *S = nullptr;
     // working-type fields (double, or float in the FP32 split)
     void *P[5], *eps, *cs, *Bc[3], *F[3][7], *E[3], *Ec[3];
@@ -37,7 +36,7 @@ struct cumc3d_ctx {
     float *sel_w = nullptr, *sel_m = nullptr, *sel_v = nullptr;   // FP32 parameters + Adam moments
     unsigned short *sel_frag = nullptr;                            // BF16 MFMA fragments
     unsigned char *mask = nullptr;                                 // 3 x G class mask
-    double2 *slot[3] = {};                                          // HLLD: carry slots per sweep (one allocation, slot[0])
+    double2 *slot[3] = {};                                          // HLLD: carry slots per sweep (in met)
     unsigned char *stale = nullptr;                                // HLL: 3 x G unassigned-face flags
     const double *sph[10] = {};   // spherical tables in met (see ArgsT), null on other geometries
     float *samp_feat = nullptr;
@@ -51,6 +50,10 @@ struct cumc3d_ctx {
     int bfac[6][12];
     cumc3d::Axis ax[3];
     bool uploaded = false, initialized = false, dt_pending = false;
+    bool dt_taken = false;        // the host has taken the CFL minimum: it starts over before the next reduction
+    cumc3d::HostScalars *pub = nullptr;   // pinned: the last step's CFL minimum
+    double *dlog = nullptr;       // cumc3d_run's dt log
+    int dlog_cap = 0;
     int next_stage = 1;           // cumc3d_stage: the stage that runs next (1 between steps)
     // timing
     bool timing = false;
@@ -194,7 +197,7 @@ template <class W> __global__ __launch_bounds__(256) void k_finddt(ArgsT<W> a) {
         dtloc = cfl_dt_rt(a, j, k, l, a.cs[c], a.P[0][c], v, b);
     }
     dtloc = block_min_f64(dtloc, a.S);
-    if (threadIdx.x == 0) atomicMin(&a.S->dtmin_bits, (unsigned long long)__double_as_longlong(dtloc));
+    if (threadIdx.x == 0) fold_dt(a.S, dtloc);
 }
 
 // FIND_DIVB (mhd_module.f90:133-189) as a max reduction on bit patterns
@@ -223,7 +226,7 @@ template <class W> __global__ __launch_bounds__(256) void k_divb(ArgsT<W> a, uns
     // max of non-negative doubles == max of their bit patterns
     unsigned long long bits = (unsigned long long)__double_as_longlong(d);
     bits = block_max_u64(bits);
-    if (threadIdx.x == 0) atomicMax(out, bits);
+    if (threadIdx.x == 0 && bits > __hip_atomic_load(out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(out, bits);
 }
 
 // ---------------------------------------------------------------------------
@@ -406,7 +409,7 @@ template <class W> static void spatial_t(cumc3d_ctx *x, double *lrk) {
     stage_update<W>(x, a, 0, dim3(nblk((long)x->nx * x->ny * x->nz)));
 }
 
-template <class W> static void run_stage_t(cumc3d_ctx *x, int stage) {
+template <class W> static void run_stage_t(cumc3d_ctx *x, int stage, HostScalars *pub) {
     hipStream_t st = x->stream;
     ArgsT<W> a = make_args<W>(x);
     const long nn = (long)x->nx * x->ny * x->nz;
@@ -415,6 +418,7 @@ template <class W> static void run_stage_t(cumc3d_ctx *x, int stage) {
     tmark(x, 5);
     x->cur = 1 - x->cur;
     ArgsT<W> g = make_args<W>(x);
+    g.pub = pub;
     stage_ghost<W>(x, g);
     tmark(x, 6);
     if (x->timing && x->tstage < TSTAGES) x->tstage += 1;
@@ -475,7 +479,7 @@ template <class W> static void sel_collect_t(cumc3d_ctx *x, int stride, unsigned
 // sweeps, selector) and fp32_state.hip (FINDDT, the layout kernels and the
 // initial update).
 namespace f32 {
-void run_stage(cumc3d_ctx *x, int stage);
+void run_stage(cumc3d_ctx *x, int stage, HostScalars *pub);
 void spatial(cumc3d_ctx *x, double *lrk);
 void sel_infer(cumc3d_ctx *x);
 void sel_collect(cumc3d_ctx *x, int stride, unsigned seed, float t1, float t2);

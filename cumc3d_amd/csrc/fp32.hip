@@ -11,7 +11,7 @@
 namespace cumc3d {
 namespace f32 {
 
-void run_stage(cumc3d_ctx *x, int stage) { run_stage_t<float>(x, stage); }
+void run_stage(cumc3d_ctx *x, int stage, HostScalars *pub) { run_stage_t<float>(x, stage, pub); }
 
 void spatial(cumc3d_ctx *x, double *lrk) { spatial_t<float>(x, lrk); }
 
