@@ -257,7 +257,11 @@ template <class W> static ArgsT<W> make_args(cumc3d_ctx *x) {
     a.rt_gravity = x->d.rt_gravity;
     a.bn_mode = x->d.hlld_bn_mode;
     for (int i = 0; i < 6; ++i) a.bc[i] = x->d.boundary_flag[i];
-    memcpy(a.bfac, x->bfac, sizeof(a.bfac));
+    for (int s = 0; s < 6; ++s) {
+        a.neg[s] = 0;
+        for (int v = 1; v < 12; ++v)
+            if (x->d.boundary_flag[s] >= 2 && x->bfac[s][v] < 0) a.neg[s] |= 1u << v;
+    }
     a.NX = x->NX; a.NY = x->NY; a.G = x->G;
     a.g1 = x->d.ggas - 1.0;
     a.cfl = x->d.cfl;
