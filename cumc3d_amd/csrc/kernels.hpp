@@ -445,6 +445,15 @@ template <class A> __device__ __forceinline__ void settle_carry(const A &a) {
     for (int d = 0; d < 3; ++d) a.S->carry[d] = c[d];
 }
 
+// The next lane's value (lane 63 keeps its own): a DPP move (wave_shl:1) per
+// 32 bits, where a shuffle goes through LDS.
+__device__ __forceinline__ int next_lane(int v) { return __builtin_amdgcn_update_dpp(v, v, 0x130, 0xf, 0xf, false); }
+__device__ __forceinline__ float next_lane(float v) { return __int_as_float(next_lane(__float_as_int(v))); }
+__device__ __forceinline__ double next_lane(double v) {
+    const long long b = __double_as_longlong(v);
+    return __longlong_as_double((long long)next_lane((int)(b >> 32)) << 32 | (unsigned)next_lane((int)b));
+}
+
 // x sweep.  The (nx+2) cells j=0..nx+1 of every row are laid end to end; each
 // 64-lane wave reconstructs 64 consecutive cells and solves the 63 interfaces
 // between them, taking the right neighbour's left face with a lane shuffle.
@@ -455,6 +464,9 @@ template <class A> __device__ __forceinline__ void settle_carry(const A &a) {
 // one of the ~68k blocks of a 256^3 sweep with many double-star interfaces
 // raised the maximum, and the atomics on the one address serialised: FP32
 // TVD-MC x sweep 0.79 ms against 0.39 ms for the z sweep on turbulence.)
+// The cell's indices come from 32-bit divisions and the neighbour's face by DPP
+// moves: with 64-bit divisions and shuffles through LDS the sweep took, at
+// 128^3 FP64 PPM, 144 us (140), at 256^3 FP32 PPM 367 (342), TVD-MC 285 (281).
 // The single-precision selector sweep is held at 5 waves per SIMD (86
 // VGPRs, 0.41 ms at 256^3).  Left to itself the compiler gives it 112 VGPRs
 // and 4 waves (0.47 ms); at 6 waves it spills (0.44 ms).
@@ -462,32 +474,32 @@ template <class T, int R, int S>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && R == RSEL ? 5 : 1)))
 void k_flux_x(ArgsT<T> a) {
     if (!a.S->active) return;
-    const int lane = threadIdx.x & 63;
-    const long nwaves = (long)gridDim.x * (blockDim.x >> 6);
-    const long wave = nwaves - 1 - (((long)blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-    const long g = wave * 63 + lane;
-    const long RL = a.nx + 2;
-    const long gtot = RL * a.ny * a.nz;
+    // all positions are below 2^30 (a field stays below 4 GiB)
+    const unsigned lane = threadIdx.x & 63;
+    const unsigned wave = gridDim.x * 4 - 1 - (blockIdx.x * 4 + (threadIdx.x >> 6));
+    const unsigned g = wave * 63 + lane;
+    const unsigned RL = a.nx + 2;
+    const unsigned gtot = RL * (unsigned)a.ny * (unsigned)a.nz;
     const bool live = g < gtot;
     int j = 0, k = 1, l = 1;
     if (live) {
-        long r = g / RL;
+        const unsigned r = g / RL, z = r / (unsigned)a.ny;
         j = (int)(g - r * RL);
-        k = 1 + (int)(r % a.ny);
-        l = 1 + (int)(r / a.ny);
+        k = 1 + (int)(r - z * (unsigned)a.ny);
+        l = 1 + (int)z;
     }
     Face<T> fm, fp;
     if (live) recon_at<T, R, 0, false>(a, j, k, l, 1, fm, fp);
     Face<T> nm;
-    nm.rho = __shfl_down(fm.rho, 1, 64);
-    nm.v[0] = __shfl_down(fm.v[0], 1, 64);
-    nm.v[1] = __shfl_down(fm.v[1], 1, 64);
-    nm.v[2] = __shfl_down(fm.v[2], 1, 64);
-    nm.p = __shfl_down(fm.p, 1, 64);
-    nm.bt1 = __shfl_down(fm.bt1, 1, 64);
-    nm.bt2 = __shfl_down(fm.bt2, 1, 64);
-    nm.eps = __shfl_down(fm.eps, 1, 64);
-    nm.cs = __shfl_down(fm.cs, 1, 64);
+    nm.rho = next_lane(fm.rho);
+    nm.v[0] = next_lane(fm.v[0]);
+    nm.v[1] = next_lane(fm.v[1]);
+    nm.v[2] = next_lane(fm.v[2]);
+    nm.p = next_lane(fm.p);
+    nm.bt1 = next_lane(fm.bt1);
+    nm.bt2 = next_lane(fm.bt2);
+    nm.eps = next_lane(fm.eps);
+    nm.cs = next_lane(fm.cs);
     unsigned serial = 0;
     __shared__ T left[S == 3 ? 2 : 1][256];   // carry of the thread's interface
     if (live && lane < 63 && j <= a.nx && g + 1 < gtot) {

@@ -84,16 +84,18 @@ template <> struct Den<double> {
     }
     __device__ __forceinline__ double tiny(double n) const {
         const bool low = __builtin_fabs(n) < 0x1p-900;
-        const double m = __builtin_amdgcn_ldexp(n, low ? 128 : 0);
+        const double m = n * (low ? 0x1p128 : 1.0);
         const double q = m * y;
         return __builtin_amdgcn_div_fixup(__builtin_amdgcn_div_fmas(__builtin_fma(-d, q, m), y, q, low), d, n);
     }
 };
 // n / 3.  The residual n - 3q is a multiple of n's last denormal place, so it
-// is exact for every n and no scaling is needed.
+// is exact for every n and no scaling is needed; taken as -(3q - n) it keeps
+// the sign of a zero without v_div_fixup.  An infinite n gives NaN: its one
+// caller's WENO weights are NaN then (inf / inf) whatever this returns.
 __device__ __forceinline__ double third(double n) {
     const double q = n * (1.0 / 3.0);
-    return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-3.0, q, n), 1.0 / 3.0, q), 3.0, n);
+    return __builtin_fma(-__builtin_fma(3.0, q, -n), 1.0 / 3.0, q);
 }
 __device__ __forceinline__ float third(float n) { return n / 3.0f; }
 __device__ __forceinline__ double sqrtS(double a) {
