@@ -22,11 +22,15 @@ LIB = os.path.join(HERE, "libcumc3d_hip.so")
 # (compare, select and two multiplies) the short divide keeps for
 # denominators beyond 2^96, and shares the reciprocal of a denominator
 # between divides.  The state unit (fp32_state.hip: update, ghost fill,
-# FINDDT) keeps IEEE division for its double arithmetic.  The FP64 unit may
-# do none of these.
+# FINDDT) keeps IEEE division for its double arithmetic.  The sweeps contract
+# within an expression only (=on): with =fast, which also fuses across
+# expressions as the optimizer finds them, two kernels of one scheme (the plain
+# and the selector's) rounded differently; the sweeps' times are within 1.5%.
+# The FP64 unit may do none of these.
 FP32_FLAGS = ["-ffp-contract=fast", "-fno-hip-fp32-correctly-rounded-divide-sqrt", "-fgpu-flush-denormals-to-zero"]
 SOURCES = [(os.path.join(HERE, "csrc", "capi.hip"), []),
-           (os.path.join(HERE, "csrc", "fp32.hip"), FP32_FLAGS + ["-fapprox-func", "-freciprocal-math"]),
+           (os.path.join(HERE, "csrc", "fp32.hip"),
+            FP32_FLAGS + ["-ffp-contract=on", "-fapprox-func", "-freciprocal-math"]),
            (os.path.join(HERE, "csrc", "fp32_state.hip"), FP32_FLAGS)]
 DEPS = [os.path.join(HERE, "csrc", f) for f in ("kernels.hpp", "physics.hpp", "selector.hpp", "context.hpp")] + \
        [os.path.join(ROOT, "include", "cumc3d_hip.h")]

@@ -30,6 +30,8 @@ template <class T> __device__ __forceinline__ T fmin_zero(T a) {
 template <class T> __device__ __forceinline__ T fabsT(T a) { return __builtin_fabs(a); }
 __device__ __forceinline__ float fabsT(float a) { return __builtin_fabsf(a); }
 __device__ __forceinline__ float fsign1(float b) { return __builtin_copysignf(1.0f, b); }
+__device__ __forceinline__ double fmaT(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ __forceinline__ float fmaT(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ double sqrtT(double a) { return __builtin_sqrt(a); }
 __device__ __forceinline__ float sqrtT(float a) { return __builtin_sqrtf(a); }
 
@@ -97,7 +99,6 @@ __device__ __forceinline__ double third(double n) {
     const double q = n * (1.0 / 3.0);
     return __builtin_fma(-__builtin_fma(3.0, q, -n), 1.0 / 3.0, q);
 }
-__device__ __forceinline__ float third(float n) { return n / 3.0f; }
 __device__ __forceinline__ double sqrtS(double a) {
     const double y = __builtin_amdgcn_rsq(a);
     double h = 0.5 * y, s = a * y;
@@ -222,63 +223,61 @@ __device__ __forceinline__ void recon_ppm(const T *__restrict__ w, T vm2, T vm1,
 
 // WENO-Z, q=2, eps=1e-40 (weno_module.f90:315-408); w = 10 weights of
 // WENO_INTERPOLANT.  In single precision eps is 1e-30 (1e-40 is below the
-// normal range) and tau5/(eps+beta) is capped at 1e18 so that its square
-// stays finite; both change nothing unless a smoothness indicator is within
-// 18 decades of zero while tau5 is not.
-template <class T> __device__ __forceinline__ T weno_ratio(T tau5, T sp, T b) {
-    T q = Den<T>(sp + b)(tau5);
-    if constexpr (sizeof(T) == 4) q = fmin2(q, T(1.0e18));
-    return q;
+// normal range) and tau5/(eps+beta) is capped at 4e17 so that its square times
+// a face value stays finite; both change nothing unless a smoothness indicator
+// is within 17 decades of zero while tau5 is not.
+// The face from the candidates P (three times the faces of the sub-stencils)
+// and the smoothness indicators B.
+__device__ __forceinline__ double weno_face(double P1, double P2, double P3, double B1, double B2, double B3) {
+    const double sp = 1.0e-40, tau5 = fabsT(B1 - B3);
+    double q = Den<double>(sp + B1)(tau5);
+    const double w1 = (1.0 / 10.0) * (1.0 + q * q);
+    q = Den<double>(sp + B2)(tau5);
+    const double w2 = (6.0 / 10.0) * (1.0 + q * q);
+    q = Den<double>(sp + B3)(tau5);
+    const double w3 = (3.0 / 10.0) * (1.0 + q * q);
+    return Den<double>(w1 + w2 + w3)(w1 * third(P1) + w2 * third(P2) + w3 * third(P3));
 }
-template <class T>
-__device__ __forceinline__ T weno_face(T P1, T P2, T P3, T B1, T B2, T B3) {
-    const T sp = sizeof(T) == 4 ? T(1.0e-30) : T(1.0e-40);
-    const T g1 = T(1.0 / 10.0), g2 = T(6.0 / 10.0), g3 = T(3.0 / 10.0);
-    T tau5 = fabsT(B1 - B3);
-    T q = weno_ratio(tau5, sp, B1);
-    T w1 = g1 * (T(1) + q * q);
-    q = weno_ratio(tau5, sp, B2);
-    T w2 = g2 * (T(1) + q * q);
-    q = weno_ratio(tau5, sp, B3);
-    T w3 = g3 * (T(1) + q * q);
-    return Den<T>(w1 + w2 + w3)(w1 * P1 + w2 * P2 + w3 * P3);
+// Single precision: weights relative to the middle one, y2 = 1/(eps + B2)
+__device__ __forceinline__ float weno_face(float P1, float P2, float P3, float B1, float y2, float B3) {
+    const float tau5 = fabsT(B1 - B3), cap = 4.0e17f;
+    const float q1 = fmin2(tau5 / B1, cap), q2 = fmin2(tau5 * y2, cap), q3 = fmin2(tau5 / B3, cap);
+    const float w1 = fmaT(q1 * float(1.0 / 6.0), q1, float(1.0 / 6.0)), w2 = fmaT(q2, q2, 1.0f),
+                w3 = fmaT(q3 * 0.5f, q3, 0.5f);
+    return fmaT(w1, P1, fmaT(w2, P2, w3 * P3)) / (3.0f * (w1 + w2 + w3));
 }
 
+// The reference's sums with common powers of two taken out of t and s (beta =
+// 13/12 t^2 + s^2/4 = 13/3 (t/2)^2 + (s/2)^2) and products by powers of two
+// fused into the additions: neither changes a bit.  What bounds a WENO-Z sweep
+// is VALU issue.  Per variable this takes 72 operations to the indicators
+// instead of 97 (double precision); in single precision the two faces also
+// share the middle indicator, which differs in rounding only.  256^3, HLLD,
+// x / y / z sweep: FP64 1.54 / 1.51 / 1.56 -> 1.49 / 1.42 / 1.49 ms, FP32
+// 0.54 / 0.61 / 0.60 -> 0.48 / 0.53 / 0.54 ms.
 template <class T>
 __device__ __forceinline__ void recon_weno(const T *__restrict__ w, T vm2, T vm1, T vc, T vp1, T vp2, T &vm_out,
                                            T &vp_out) {
-    const T r1 = T(13.0 / 12.0), r2 = T(1.0 / 4.0);
-    T U01 = w[0] * vc + w[1] * vp1;
-    T U12 = w[2] * vp1 + w[3] * vp2;
-    T U10 = w[4] * vm1 + w[5] * vc;
-    T U21 = w[6] * vm2 + w[7] * vm1;
-    T U00 = vm1 + w[8] * (vm1 - vm2);
-    T U11 = vp1 + w[9] * (vp1 - vp2);
-    T t, s;
-    {
-        T P1 = third(T(6) * vc - T(1) * U10 - T(2) * U00);
-        T P2 = third(-T(1) * U10 + T(2) * vc + T(2) * U01);
-        T P3 = third(T(2) * U01 + T(2) * vp1 - T(1) * U12);
-        t = T(2) * U10 - T(2) * U00; s = T(4) * vc - T(2) * U10 - T(2) * U00;
-        T B1 = r1 * (t * t) + r2 * (s * s);
-        t = T(2) * U10 - T(4) * vc + T(2) * U01; s = -T(2) * U10 + T(2) * U01;
-        T B2 = r1 * (t * t) + r2 * (s * s);
-        t = T(2) * U01 - T(4) * vp1 + T(2) * U12; s = -T(6) * U01 + T(8) * vp1 - T(2) * U12;
-        T B3 = r1 * (t * t) + r2 * (s * s);
-        vp_out = weno_face(P1, P2, P3, B1, B2, B3);
-    }
-    {
-        T P1 = third(T(6) * vc - T(1) * U01 - T(2) * U11);
-        T P2 = third(-T(1) * U01 + T(2) * vc + T(2) * U10);
-        T P3 = third(T(2) * U10 + T(2) * vm1 - T(1) * U21);
-        t = T(2) * U01 - T(2) * U11; s = T(4) * vc - T(2) * U01 - T(2) * U11;
-        T B1 = r1 * (t * t) + r2 * (s * s);
-        t = T(2) * U01 - T(4) * vc + T(2) * U10; s = T(2) * U01 - T(2) * U10;
-        T B2 = r1 * (t * t) + r2 * (s * s);
-        t = T(2) * U10 - T(4) * vm1 + T(2) * U21; s = T(8) * vm1 - T(6) * U10 - T(2) * U21;
-        T B3 = r1 * (t * t) + r2 * (s * s);
-        vm_out = weno_face(P1, P2, P3, B1, B2, B3);
-    }
+    const T r = T(13.0 / 12.0) * T(4);
+    const T U01 = w[0] * vc + w[1] * vp1;
+    const T U12 = w[2] * vp1 + w[3] * vp2;
+    const T U10 = w[4] * vm1 + w[5] * vc;
+    const T U21 = w[6] * vm2 + w[7] * vm1;
+    const T U00 = vm1 + w[8] * (vm1 - vm2);
+    const T U11 = vp1 + w[9] * (vp1 - vp2);
+    const T X = fmaT(T(2), vc, -U10), Y = fmaT(T(2), vc, -U01);
+    // single precision: eps enters with the indicator, where it is free
+    auto sq = [](T s) { return sizeof(T) == 4 ? fmaT(s, s, T(1.0e-30)) : s * s; };
+    auto beta = [&](T t, T s2) { return r * (t * t) + s2; };
+    const T s2 = sq(U01 - U10);
+    const T B1p = beta(U10 - U00, sq(X - U00)), B1m = beta(U01 - U11, sq(Y - U11));
+    const T B3p = beta(fmaT(T(-2), vp1, U01) + U12, sq(fmaT(T(4), vp1, -(T(3) * U01)) - U12));
+    const T B3m = beta(fmaT(T(-2), vm1, U10) + U21, sq(fmaT(T(4), vm1, -(T(3) * U10)) - U21));
+    T B2p = beta(U01 - X, s2), B2m;
+    if constexpr (sizeof(T) == 4) B2m = B2p = T(1) / B2p;   // the two differ in rounding only
+    else B2m = beta(U10 - Y, s2);
+    vp_out = weno_face(fmaT(T(-2), U00, T(6) * vc - U10), fmaT(T(2), U01, X), fmaT(T(2), U01 + vp1, -U12), B1p, B2p, B3p);
+    vm_out = weno_face(fmaT(T(-2), U11, T(6) * vc - U01), fmaT(T(2), U10, Y), fmaT(T(2), U10 + vm1, -U21), B1m, B2m, B3m);
 }
 
 // Scheme ids as in the build descriptor: 0 minmod, 1 van Leer, 2 MC, 3 PPM, 4 WENO-Z.
