@@ -181,14 +181,16 @@ static bool setup_bfac(const int *bf, int bfac[6][12]) {
 // (tvd_module.f90:42-53, ppmc_module.f90:91-145, weno_module.f90:117-149)
 static void weights(int recon, const std::vector<double> &dd, int n, std::vector<double> &w) {
     w.assign((size_t)(n + 7) * NW, 0.0);
-    auto D = [&](int j) { return dd[j + 3]; };
+    auto D = [&](int j) { return j + 3 < (int)dd.size() ? dd[j + 3] : 0.0; };
     if (recon <= 2) {
         for (int j = -1; j <= n + 2; ++j) {
             w[(j + 3) * NW + 0] = (D(j) + D(j + 1)) / D(j);
             w[(j + 3) * NW + 1] = (D(j) + D(j - 1)) / D(j);
         }
     } else if (recon == 3) {
-        for (int j = 0; j <= n + 1; ++j) {
+        // cells -1 and n+2, for the x sweep: the slope weights (10, 11) and,
+        // of cell -1, the upper edge's (4 to 7); their others lack a width
+        for (int j = -1; j <= n + 2; ++j) {
             double dm2 = D(j - 2), dm1 = D(j - 1), dc = D(j), dp1 = D(j + 1), dp2 = D(j + 2);
             double a1R = dc / (dc + dp1), a1L = dm1 / (dm1 + dc);
             double aR = 2.0 * dp1 * dc / (dp1 + dc), aL = 2.0 * dc * dm1 / (dc + dm1);

@@ -313,12 +313,13 @@ static int nseg_for(const cumc3d_ctx *x, int nx, int na, int nd) {
 // ---------------------------------------------------------------------------
 // flux dispatch over (reconstruction, Riemann solver)
 // ---------------------------------------------------------------------------
-// Grid of the sweep along D: x by waves of 63 interfaces (k_flux_x), y and z by
+// Grid of the sweep along D: x by waves of 63 or 61 interfaces (k_flux_x), y and z by
 // planes across the sweep axis and march segments (k_flux_yz).
 static dim3 sweep_grid(const cumc3d_ctx *x, int D, int &nseg) {
     nseg = 1;
     if (D == 0) {
-        const long waves = ((long)(x->nx + 2) * x->ny * x->nz + 62) / 63 + 1;
+        const int h = x_halo(x->sel_on ? RSEL : x->d.recon), per = 63 - 2 * h;
+        const long waves = ((long)(x->nx + 2 + 2 * h) * x->ny * x->nz + per - 1) / per + 1;
         return dim3((unsigned)((waves * 64 + 255) / 256));
     }
     const int na = D == 1 ? x->nz : x->ny, nd = D == 1 ? x->ny : x->nz;

@@ -193,34 +193,37 @@ __device__ __forceinline__ void recon_tvd(T cf, T cb, T vm, T vc, T vp, T &vm_ou
 }
 
 // PPM without steepening/flattening (ppmc_module.f90:359-464); w = 14
-// interpolation weights of PPM_INTERPOLANT.
-template <class T>
-__device__ __forceinline__ void recon_ppm(const T *__restrict__ w, T vm2, T vm1, T vc, T vp1, T vp2, T &vm_out,
-                                          T &vp_out) {
-    T deltap1 = w[12] * (vp2 - vp1) + w[13] * (vp1 - vc);
-    T deltac = w[10] * (vp1 - vc) + w[11] * (vc - vm1);
-    T deltam1 = w[8] * (vc - vm1) + w[9] * (vm1 - vm2);
-    T dmc = T(0), dmp1 = T(0), dmm1 = T(0);
-    if ((vp1 - vc) * (vc - vm1) > T(0))
-        dmc = fmin2(fmin2(fabsT(deltac), T(2) * fabsT(vc - vm1)), T(2) * fabsT(vc - vp1)) * fsign1(deltac);
-    if ((vp2 - vp1) * (vp1 - vc) > T(0))
-        dmp1 = fmin2(fmin2(fabsT(deltap1), T(2) * fabsT(vp1 - vc)), T(2) * fabsT(vp1 - vp2)) * fsign1(deltap1);
-    if ((vc - vm1) * (vm1 - vm2) > T(0))
-        dmm1 = fmin2(fmin2(fabsT(deltam1), T(2) * fabsT(vm1 - vm2)), T(2) * fabsT(vm1 - vc)) * fsign1(deltam1);
-    T vp = vc + w[4] * (vp1 - vc) + w[5] * (vp1 - vc) + w[6] * dmp1 + w[7] * dmc;
-    T vm = vm1 + w[0] * (vc - vm1) + w[1] * (vc - vm1) + w[2] * dmc + w[3] * dmm1;
-    T vl = vm, vr = vp;
-    if ((vr - vc) * (vc - vl) <= T(0)) {
-        vp = vc;
-        vm = vc;
-    } else {
-        if ((vr - vl) * (vl - T(3) * vc + T(2) * vr) < T(0)) vm = T(3) * vc - T(2) * vr;
-        if ((vp - vm) * (T(3) * vc - T(2) * vl - vr) < T(0)) vp = T(3) * vc - T(2) * vl;
-    }
-    vm_out = vm;
-    vp_out = vp;
+// interpolation weights of PPM_INTERPOLANT, in pieces that neighbouring cells
+// can share: the limited slope of a cell, the value at its upper edge (the
+// lower edge of the next cell), and the limiter of the two edges.  The weights
+// of a shared piece are the same expressions of the same widths seen from
+// either cell, so it has the same bits; products by 2 fused into a sum too.
+template <class T> __device__ __forceinline__ T ppm_slope(T wb, T wa, T a, T b) {
+    const T d = wb * b + wa * a;
+    const T m = __builtin_elementwise_min(fabsT(d), T(2) * __builtin_elementwise_min(fabsT(a), fabsT(b)));
+    return b * a > T(0) ? __builtin_elementwise_copysign(m, d) : T(0);
 }
-
+// upper edge of cell c: w = its weights 4..7, b = v(c+1) - v(c), dc and dp the slopes of c and c+1
+template <class T> __device__ __forceinline__ T ppm_edge(const T *w, T vc, T b, T dc, T dp) {
+    return vc + w[0] * b + w[1] * b + w[2] * dp + w[3] * dc;
+}
+template <class T> __device__ __forceinline__ void ppm_limit(T vc, T vl, T vr, T &vm_out, T &vp_out) {
+    const T c3 = T(3) * vc, lo = fmaT(T(-2), vr, c3), hi = fmaT(T(-2), vl, c3);
+    const T vm = (vr - vl) * fmaT(T(2), vr, vl - c3) < T(0) ? lo : vl;
+    const T vp = (vr - vm) * (hi - vr) < T(0) ? hi : vr;
+    const bool flat = (vr - vc) * (vc - vl) <= T(0);
+    vm_out = flat ? vc : vm;
+    vp_out = flat ? vc : vp;
+}
+// Both edges of a cell from its whole stencil, and the slope of the next cell
+template <class T>
+__device__ __forceinline__ void ppm_edges(const T *__restrict__ w, const T s[5], T &low, T &high, T &dp) {
+    const T a = s[2] - s[1], b = s[3] - s[2];
+    const T dm = ppm_slope(w[8], w[9], s[1] - s[0], a), dc = ppm_slope(w[10], w[11], a, b);
+    dp = ppm_slope(w[12], w[13], b, s[4] - s[3]);
+    low = ppm_edge(w, s[1], a, dm, dc);
+    high = ppm_edge(w + 4, s[2], b, dc, dp);
+}
 // WENO-Z, q=2, eps=1e-40 (weno_module.f90:315-408); w = 10 weights of
 // WENO_INTERPOLANT.  In single precision eps is 1e-30 (1e-40 is below the
 // normal range) and tau5/(eps+beta) is capped at 4e17 so that its square times
@@ -284,7 +287,11 @@ __device__ __forceinline__ void recon_weno(const T *__restrict__ w, T vm2, T vm1
 template <class T, int R>
 __device__ __forceinline__ void recon1(const T *__restrict__ w, const T s[5], T &vm_out, T &vp_out) {
     if constexpr (R <= 2) recon_tvd<T, R>(w[0], w[1], s[1], s[2], s[3], vm_out, vp_out);
-    else if constexpr (R == 3) recon_ppm<T>(w, s[0], s[1], s[2], s[3], s[4], vm_out, vp_out);
+    else if constexpr (R == 3) {
+        T low, high, dp;
+        ppm_edges(w, s, low, high, dp);
+        ppm_limit(s[2], low, high, vm_out, vp_out);
+    }
     else recon_weno<T>(w, s[0], s[1], s[2], s[3], s[4], vm_out, vp_out);
 }
 
@@ -296,14 +303,8 @@ template <class T> struct Face {
     T rho, v[3], p, bt1, bt2, eps, cs;
 };
 
-template <class T, int R>
-__device__ __forceinline__ void recon_cell(const T *__restrict__ w, const T st[7][5], T g1, Face<T> &fm,
-                                           Face<T> &fp) {
-    recon1<T, R>(w, st[0], fm.rho, fp.rho);
-    recon1<T, R>(w, st[1], fm.v[0], fp.v[0]);
-    recon1<T, R>(w, st[2], fm.v[1], fp.v[1]);
-    recon1<T, R>(w, st[3], fm.v[2], fp.v[2]);
-    recon1<T, R>(w, st[4], fm.p, fp.p);
+// epsilon and the sound speed at both faces
+template <class T> __device__ __forceinline__ void face_eos(T g1, Face<T> &fm, Face<T> &fp) {
     if constexpr (sizeof(T) == 4) {
         // single precision: one reciprocal per face.  eps = (p / rho) / g1 and
         // eps g1 + rho g1 p / rho^2 = (g1 + 1) p / rho, the ideal-gas c_s^2
@@ -319,6 +320,17 @@ __device__ __forceinline__ void recon_cell(const T *__restrict__ w, const T st[7
         fm.cs = eos_cs(g1, fm.p, fm.rho, fm.eps);
         fp.cs = eos_cs(g1, fp.p, fp.rho, fp.eps);
     }
+}
+
+template <class T, int R>
+__device__ __forceinline__ void recon_cell(const T *__restrict__ w, const T st[7][5], T g1, Face<T> &fm,
+                                           Face<T> &fp) {
+    recon1<T, R>(w, st[0], fm.rho, fp.rho);
+    recon1<T, R>(w, st[1], fm.v[0], fp.v[0]);
+    recon1<T, R>(w, st[2], fm.v[1], fp.v[1]);
+    recon1<T, R>(w, st[3], fm.v[2], fp.v[2]);
+    recon1<T, R>(w, st[4], fm.p, fp.p);
+    face_eos(g1, fm, fp);
     recon1<T, R>(w, st[5], fm.bt1, fp.bt1);
     recon1<T, R>(w, st[6], fm.bt2, fp.bt2);
 }
