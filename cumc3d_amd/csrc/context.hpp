@@ -314,7 +314,11 @@ static int nseg_for(const cumc3d_ctx *x, int nx, int na, int nd) {
 // flux dispatch over (reconstruction, Riemann solver)
 // ---------------------------------------------------------------------------
 // Grid of the sweep along D: x by waves of 63 or 61 interfaces (k_flux_x), y and z by
-// planes across the sweep axis and march segments (k_flux_yz).
+// planes across the sweep axis and march segments (k_flux_yz); flat: the
+// selector's y and z sweeps where a plane is no whole number of waves.
+static bool sweep_flat(const cumc3d_ctx *x, int D) {
+    return x->sel_on && D > 0 && ((long)x->nx * (D == 1 ? x->nz : x->ny)) % 64 != 0;
+}
 static dim3 sweep_grid(const cumc3d_ctx *x, int D, int &nseg) {
     nseg = 1;
     if (D == 0) {
@@ -324,6 +328,7 @@ static dim3 sweep_grid(const cumc3d_ctx *x, int D, int &nseg) {
     }
     const int na = D == 1 ? x->nz : x->ny, nd = D == 1 ? x->ny : x->nz;
     nseg = nseg_for(x, x->nx, na, nd);
+    if (sweep_flat(x, D)) return dim3(nblk((long)x->nx * na * nseg));
     return dim3(nblk((long)x->nx * na), nseg);
 }
 
@@ -331,9 +336,18 @@ template <class W, int R, int S>
 static void launch_sweep_rs(cumc3d_ctx *x, const ArgsT<W> &a, int D, hipStream_t st) {
     int ns;
     const dim3 grid = sweep_grid(x, D, ns);
+    auto yz = D == 1 ? k_flux_yz<W, R, S, 1> : k_flux_yz<W, R, S, 2>;
+    if constexpr (R == RSEL) {
+        if (sweep_flat(x, D)) yz = D == 1 ? k_flux_yz<W, R, S, 1, true> : k_flux_yz<W, R, S, 2, true>;
+    }
     if (D == 0) hipLaunchKernelGGL((k_flux_x<W, R, S>), grid, dim3(256), 0, st, a);
-    else if (D == 1) hipLaunchKernelGGL((k_flux_yz<W, R, S, 1>), grid, dim3(256), 0, st, a, ns);
-    else hipLaunchKernelGGL((k_flux_yz<W, R, S, 2>), grid, dim3(256), 0, st, a, ns);
+    else hipLaunchKernelGGL(yz, grid, dim3(256), 0, st, a, ns);
+    if constexpr (R == RSEL && S == 3) {
+        if (a.bn_mode != 2) return;
+        if (D == 0) hipLaunchKernelGGL((k_carry_own<W, 0>), dim3(1), dim3(64), 0, st, a);
+        else if (D == 1) hipLaunchKernelGGL((k_carry_own<W, 1>), dim3(1), dim3(64), 0, st, a);
+        else hipLaunchKernelGGL((k_carry_own<W, 2>), dim3(1), dim3(64), 0, st, a);
+    }
 }
 
 template <class W, int R>

@@ -622,10 +622,16 @@ __device__ __forceinline__ void ppm_next(const ArgsT<T> &a, long c, int i, long 
 // HLLD + WENO-Z: 2.05 / 1.95 -> 1.56 / 1.56 ms.  In single precision the face
 // stays in registers for the fixed schemes: from LDS, TVD-MC took 0.360 against
 // 0.353 ms and PPM 0.495 against 0.474 ms (the selector 0.400 against 0.467).
-template <class T, int R, int S, int D>
+// FLAT (the selector, where the planes are no whole number of waves): the
+// segments too are laid end to end over the threads.  A wave reconstructs all
+// its cells by its highest class, so which cells share a wave is part of the
+// selector's result: 64 consecutive ones of (segment, plane).  Where planes are
+// whole waves the two layouts put the same cells in a wave, and the segment per
+// block row gives it one weight set.
+template <class T, int R, int S, int D, bool FLAT = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 3 : 1))) void k_flux_yz(ArgsT<T> a, int nseg) {
     if (!a.S->active) return;
-    const unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
+    const unsigned thread = blockIdx.x * blockDim.x + threadIdx.x;
     const int na = (D == 1) ? a.nz : a.ny;    // the other transverse axis
     const int nd = (D == 1) ? a.ny : a.nz;    // sweep axis
     unsigned serial = 0;
@@ -633,10 +639,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
     __shared__ T pk[R == 3 ? 14 : 1][256];
     __shared__ T kept[lds ? 9 : 1][256];
     __shared__ T left[S == 3 ? 2 : 1][256];   // carry of the thread's last double-star interface
-    if (t < (unsigned)a.nx * (unsigned)na) {
+    const unsigned plane = (unsigned)a.nx * (unsigned)na;
+    const int s = FLAT ? (int)(thread / plane) : (int)blockIdx.y;
+    const unsigned t = FLAT ? thread - (unsigned)s * plane : thread;
+    if (t < plane && s < nseg) {
         const int o2 = 1 + (int)(t / (unsigned)a.nx);
         const int j = 1 + (int)(t - (unsigned)(o2 - 1) * (unsigned)a.nx);
-        const int s = blockIdx.y;
         const int i0 = (int)(((long)s * (nd + 1)) / nseg);
         const int i1 = (int)(((long)(s + 1) * (nd + 1)) / nseg);
         const long st = stride<D>(a);
@@ -651,11 +659,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
         long cc = cidx(a, j, (D == 1) ? i0 : o2, (D == 1) ? o2 : i0);
         if constexpr (slide) {
             load_stencil<T, stencil_r<R>(), D>(a, cc, st, win);
-            recon_stencil<T, R, D, true>(a, cc, i0, win, fm, fp);
+            recon_stencil<T, R, D, !FLAT>(a, cc, i0, win, fm, fp);
         } else if constexpr (R == 3) {
             ppm_first<T, D>(a, cc, i0, st, pk, fm, fp);
         } else {
-            recon_at<T, R, D, true>(a, j, (D == 1) ? i0 : o2, (D == 1) ? o2 : i0, st, fm, fp);
+            recon_at<T, R, D, !FLAT>(a, j, (D == 1) ? i0 : o2, (D == 1) ? o2 : i0, st, fm, fp);
         }
         const T carry = S == 3 ? (T)carried<D>(a) : T(0);
         if constexpr (lds) keep_face(kept, fp);
@@ -669,11 +677,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
             cc += st;
             if constexpr (slide) {
                 slide_stencil<T, R, D>(a, cc, st, win);
-                recon_stencil<T, R, D, true>(a, cc, i, win, fm, fp);
+                recon_stencil<T, R, D, !FLAT>(a, cc, i, win, fm, fp);
             } else if constexpr (R == 3) {
                 ppm_next<T, D>(a, cc, i, st, pk, fm, fp);
             } else {
-                recon_at<T, R, D, true>(a, j, k, l, st, fm, fp);
+                recon_at<T, R, D, !FLAT>(a, j, k, l, st, fm, fp);
             }
             if constexpr (lds) {
                 prev = kept_face(kept);
@@ -696,6 +704,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
     if constexpr (S == 3) {
         if (a.bn_mode == 2) fold_carry(a.S, a.slot[D], D, serial, left);
     }
+}
+
+// The selector's carry: the value the last double-star interface gives when its
+// two cells take their own classes, not their wave's highest (one thread; 0
+// where that is no double star), in place of what the sweep left in the slot.
+template <class T, int D> __global__ __launch_bounds__(64) void k_carry_own(ArgsT<T> a) {
+    if (!a.S->active || threadIdx.x != 0) return;
+    const unsigned long long key = a.S->carry_key[D];
+    if (key == 0) return;
+    unsigned q = (unsigned)(key >> 32) - 1;     // serial_key<D> undone
+    const unsigned nx = a.nx + (D == 0), ny = a.ny + (D == 1), x = q % nx;
+    q /= nx;
+    const int j = (int)x + (D != 0), k = (int)(q % ny) + (D != 1), l = (int)(q / ny) + (D != 2);
+    const long st = stride<D>(a);
+    Face<T> lm, lp, rm, rp;
+    recon_at<T, RSEL, D, false>(a, j, k, l, st, lm, lp);
+    recon_at<T, RSEL, D, false>(a, j + (D == 0), k + (D == 1), l + (D == 2), st, rm, rp);
+    const T bn = (T)a.Bin[D][cidx(a, j, k, l)];
+    RiemannOut<T> o;
+    riemann<T, D, 3>(to_q<T, D>(lp, bn), to_q<T, D>(rm, bn), lp.eps, rm.eps, lp.cs, rm.cs, a.bn_mode, (T)carried<D>(a), o);
+    a.slot[D][(unsigned)key] = make_double2(o.uss_t1, o.uss_t2);
 }
 
 // ---------------------------------------------------------------------------
