@@ -613,12 +613,20 @@ int cumc3d_init(const cumc3d_desc *desc, cumc3d_ctx **out) {
         long v = atol(mt);
         if (v >= 1) x->march_threads = v;
     }
+    for (int D = 1; D < 3; ++D) {
+        const long cols = (long)x->nx * (D == 1 ? x->nz : x->ny);
+        const int n = (D == 1 ? x->ny : x->nz) + 1;
+        x->march[D - 1] = x->march_threads ? segments_of(x->march_threads, cols, n) : segments(cols, n);
+    }
     size_t slots[4] = {};
     if (d.riemann == CUMC3D_HLLD && d.hlld_bn_mode == 2)
         for (int D = 0; D < 3; ++D) {
             int ns;
-            const dim3 g = sweep_grid(x, D, ns);
-            slots[D + 1] = slots[D] + (D < d.n_dim ? (size_t)g.x * g.y : 0);
+            dim3 f;
+            const dim3 g = sweep_grid(x, D, false, ns);
+            size_t n = (size_t)g.x * g.y;
+            if (flat_grid(x, D, ns, f) && f.x > n) n = f.x;
+            slots[D + 1] = slots[D] + (D < d.n_dim ? n : 0);
         }
     const size_t wat = (hm.size() * sizeof(double) + 255) / 256 * 256;
     const size_t sat = wat + (hw.size() * wsz + 255) / 256 * 256;

@@ -29,7 +29,8 @@ struct cumc3d_ctx {
     // always double: face field (ping-pong), u_old, conserved state (FP32 split), floors
     double *B[2][3], *Uo[8], *U[5], *floors[3];
     int cur = 0;                  // B[cur] holds the current face field
-    long march_threads = 1L << 19;  // target thread count of the y/z sweeps
+    long march_threads = 0;         // y/z sweeps' thread count from CUMC3D_MARCH_THREADS (0: segments())
+    int march[2] = {1, 1};          // segments per column of the y and z sweeps
     // learned reconstruction selector
     bool sel_on = false;
     int sel_every = 1, sel_tick = 0;
@@ -298,47 +299,73 @@ template <class W> static ArgsT<W> make_args(cumc3d_ctx *x) {
 
 static inline unsigned nblk(long n, int b = 256) { return (unsigned)((n + b - 1) / b); }
 
+// As many segments of n interfaces as make `threads` threads of `cols` columns
+static int segments_of(long threads, long cols, int n) {
+    const long want = threads / cols;
+    return (int)(want < 1 ? 1 : (want > n ? n : want));
+}
 // Segments per column of the y/z sweeps: each thread marches one segment of
-// interfaces along the sweep axis, reusing the reconstruction of the cell it
-// shares with the previous interface.  About march_threads threads in flight
-// (2^19 = 8k waves by default); CUMC3D_MARCH_THREADS overrides it at init.
-static int nseg_for(const cumc3d_ctx *x, int nx, int na, int nd) {
-    long cols = (long)nx * na;
-    long want = x->march_threads / (cols > 0 ? cols : 1);
-    if (want < 1) want = 1;
-    if (want > nd + 1) want = nd + 1;
-    return (int)want;
+// the n interfaces along the sweep axis, reusing the reconstruction of the cell
+// it shares with the previous interface.  2^19 threads load the CUs evenly, but
+// each segment costs its column one more cell, most of the work where that
+// leaves one or two interfaces a segment.  A sweep is bound by VALU issue, so a
+// CU with k blocks takes k times a block's cells, its longest march and the cell
+// before it; with few blocks a CU the others wait for the fullest and latency
+// shows (`few`, measured).  Fewer segments are taken where that estimate is 3%
+// below the even load's.  Measured against 2^19 threads throughout (y / z, FP64
+// HLLD + PPM): 96x64x96 54 / 58 -> 45 / 44 us, 128x96x64 55 / 56 -> 48 / 51, 128^3
+// 142 / 117 -> 135 / 112; FP32 64^3 15.6 / 14.8 -> 14.8 / 13.8.  At 256^3 3 segments
+// instead of 8 were 3.5% slower (WENO-Z), at 192^3 13 instead of 14 3%.
+static int segments(long cols, int n) {
+    constexpr int cus = 256;
+    const double few[8] = {0.0, 1.8, 1.2, 1.05, 1.05, 1.02, 1.02, 1.02};
+    const long blocks = nblk(cols);
+    auto cost = [&](int s) {
+        const long k = (blocks * s + cus - 1) / cus;
+        return k < 8 ? few[k] * k * ((n + s - 1) / s + 1) : (double)blocks / cus * (n + s);
+    };
+    int at = segments_of(1L << 19, cols, n);
+    double best = 0.97 * cost(at);
+    for (int s = at - 1; s >= 1; --s)
+        if (cost(s) < best) {
+            best = cost(s);
+            at = s;
+        }
+    return at;
 }
 
 // ---------------------------------------------------------------------------
 // flux dispatch over (reconstruction, Riemann solver)
 // ---------------------------------------------------------------------------
 // Grid of the sweep along D: x by waves of 63 or 61 interfaces (k_flux_x), y and z by
-// planes across the sweep axis and march segments (k_flux_yz); flat: the
-// selector's y and z sweeps where a plane is no whole number of waves.
-static bool sweep_flat(const cumc3d_ctx *x, int D) {
-    return x->sel_on && D > 0 && ((long)x->nx * (D == 1 ? x->nz : x->ny)) % 64 != 0;
-}
-static dim3 sweep_grid(const cumc3d_ctx *x, int D, int &nseg) {
+// planes across the sweep axis and march segments (k_flux_yz).
+static dim3 sweep_grid(const cumc3d_ctx *x, int D, bool selector, int &nseg) {
     nseg = 1;
     if (D == 0) {
-        const int h = x_halo(x->sel_on ? RSEL : x->d.recon), per = 63 - 2 * h;
+        const int h = selector ? 0 : x_halo(x->d.recon), per = 63 - 2 * h;
         const long waves = ((long)(x->nx + 2 + 2 * h) * x->ny * x->nz + per - 1) / per + 1;
         return dim3((unsigned)((waves * 64 + 255) / 256));
     }
-    const int na = D == 1 ? x->nz : x->ny, nd = D == 1 ? x->ny : x->nz;
-    nseg = nseg_for(x, x->nx, na, nd);
-    if (sweep_flat(x, D)) return dim3(nblk((long)x->nx * na * nseg));
-    return dim3(nblk((long)x->nx * na), nseg);
+    nseg = x->march[D - 1];
+    return dim3(nblk((long)x->nx * (D == 1 ? x->nz : x->ny)), nseg);
+}
+// The selector's y or z sweep where a plane is no whole number of waves: 2^19
+// threads laid end to end (its result depends on the segments there)
+static bool flat_grid(const cumc3d_ctx *x, int D, int &nseg, dim3 &grid) {
+    const long cols = (long)x->nx * (D == 1 ? x->nz : x->ny);
+    if (D == 0 || cols % 64 == 0) return false;
+    nseg = segments_of(x->march_threads ? x->march_threads : 1L << 19, cols, (D == 1 ? x->ny : x->nz) + 1);
+    grid = dim3(nblk(cols * nseg));
+    return true;
 }
 
 template <class W, int R, int S>
 static void launch_sweep_rs(cumc3d_ctx *x, const ArgsT<W> &a, int D, hipStream_t st) {
     int ns;
-    const dim3 grid = sweep_grid(x, D, ns);
+    dim3 grid = sweep_grid(x, D, R == RSEL, ns);
     auto yz = D == 1 ? k_flux_yz<W, R, S, 1> : k_flux_yz<W, R, S, 2>;
     if constexpr (R == RSEL) {
-        if (sweep_flat(x, D)) yz = D == 1 ? k_flux_yz<W, R, S, 1, true> : k_flux_yz<W, R, S, 2, true>;
+        if (flat_grid(x, D, ns, grid)) yz = D == 1 ? k_flux_yz<W, R, S, 1, true> : k_flux_yz<W, R, S, 2, true>;
     }
     if (D == 0) hipLaunchKernelGGL((k_flux_x<W, R, S>), grid, dim3(256), 0, st, a);
     else hipLaunchKernelGGL(yz, grid, dim3(256), 0, st, a, ns);
