@@ -683,9 +683,9 @@ int cumc3d_init(const cumc3d_desc *desc, cumc3d_ctx **out) {
         for (int i = 0; i < 7; ++i) x->F[dd][i] = takew();
     for (int i = 0; i < 3; ++i) x->E[i] = takew();
     for (int i = 0; i < 3; ++i) x->Ec[i] = takew();
-    for (int b = 0; b < 2; ++b)
+    for (int b = 0; b < 3; ++b)
         for (int i = 0; i < 3; ++i) x->B[b][i] = taked();
-    for (int i = 0; i < 8; ++i) x->Uo[i] = taked();
+    for (int i = 0; i < 5; ++i) x->Uo[i] = taked();
     for (int i = 0; i < 5; ++i) x->U[i] = x->fp32 ? taked() : nullptr;
     for (int i = 0; i < 3; ++i) x->floors[i] = taked();
     if (hipMalloc(&x->S, sizeof(DevScalars)) != hipSuccess) { cleanup(); return fail(CUMC3D_ENOMEM, "scalars"); }

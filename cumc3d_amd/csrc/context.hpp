@@ -27,8 +27,9 @@ struct cumc3d_ctx {
     // working-type fields (double, or float in the FP32 split)
     void *P[5], *eps, *cs, *Bc[3], *F[3][7], *E[3], *Ec[3];
     // always double: face field (ping-pong), u_old, conserved state (FP32 split), floors
-    double *B[2][3], *Uo[8], *U[5], *floors[3];
-    int cur = 0;                  // B[cur] holds the current face field
+    double *B[3][3], *Uo[5], *U[5], *floors[3];
+    int cur = 0;                  // B[cur] holds the current face field,
+    int old = 0;                  // B[old] that of the step's start
     long march_threads = 0;         // y/z sweeps' thread count from CUMC3D_MARCH_THREADS (0: segments())
     int march[2] = {1, 1};          // segments per column of the y and z sweeps
     // learned reconstruction selector
@@ -97,6 +98,7 @@ template <class W> __global__ void k_split_prim(const double *aos, const double 
     for (int d = 0; d < 3; ++d) {
         a.Bin[d][c] = q[5 + d];
         a.Bout[d][c] = q[5 + d];
+        a.Bold[d][c] = q[5 + d];
     }
     a.eps[c] = (W)eps64[c];
     if constexpr (sizeof(W) == 4) {
@@ -274,12 +276,13 @@ template <class W> static ArgsT<W> make_args(cumc3d_ctx *x) {
     for (int d = 0; d < 3; ++d) {
         a.Bc[d] = (W *)x->Bc[d];
         a.Bin[d] = x->B[x->cur][d];
-        a.Bout[d] = x->B[1 - x->cur][d];
+        a.Bout[d] = x->B[(x->cur + 1) % 3][d];
+        a.Bold[d] = x->B[(x->cur + 2) % 3][d];
         a.E[d] = (W *)x->E[d];
         a.Ec[d] = (W *)x->Ec[d];
         for (int i = 0; i < 7; ++i) a.F[d][i] = (W *)x->F[d][i];
     }
-    for (int i = 0; i < 8; ++i) a.Uo[i] = x->Uo[i];
+    for (int i = 0; i < 5; ++i) a.Uo[i] = x->Uo[i];
     for (int i = 0; i < 5; ++i) a.U[i] = x->U[i];
     a.rfl = x->floors[0];
     a.pfl = x->floors[1];
@@ -460,10 +463,19 @@ template <class W> static void run_stage_t(cumc3d_ctx *x, int stage, HostScalars
     ArgsT<W> a = make_args<W>(x);
     const long nn = (long)x->nx * x->ny * x->nz;
     sweeps_t<W>(x, a, st, true);
+    // stage 1 writes either other buffer, stages 2 and 3 the one that holds
+    // neither the current field nor that of the step's start
+    if (stage == 1) x->old = x->cur;
+    const int in = x->cur, out = stage == 1 ? (in + 1) % 3 : 3 - in - x->old;
+    for (int d = 0; d < 3; ++d) {
+        a.Bout[d] = x->B[out][d];
+        a.Bold[d] = x->B[x->old][d];
+    }
     stage_update<W>(x, a, stage, dim3(nblk(nn)));
     tmark(x, 5);
-    x->cur = 1 - x->cur;
+    x->cur = out;
     ArgsT<W> g = make_args<W>(x);
+    for (int d = 0; d < 3; ++d) g.Bout[d] = x->B[in][d];   // an inactive step's state
     g.pub = pub;
     stage_ghost<W>(x, g);
     tmark(x, 6);

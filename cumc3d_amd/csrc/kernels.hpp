@@ -84,7 +84,8 @@ template <class W> struct ArgsT {
     W *Bc[3];               // cell-centred field (bcell)
     double *Bin[3];         // face field at stage start (prim(ibx..ibz))
     double *Bout[3];        // face field written by the update
-    double *Uo[8];          // u_old
+    double *Bold[3];        // face field at the step's start
+    double *Uo[5];          // u_old
     double *U[5];           // conserved hydro state (FP32 split only)
     W *F[3][7];             // interface fluxes: 5 hydro + 2 face EMFs
     W *E[3];                // edge EMFs efield_x/y/z
@@ -1219,31 +1220,18 @@ __device__ __forceinline__ double update_cell(const ArgsT<W> &a, int j, int k, i
             if (l == 1) o[8 * (c - sz) + 7] = lB_z<G>(a, j, k, ey_mz, ey_mxmz, ex_mz, ex_mymz);
             return 1.0e5;
         }
-        // all six face loads first: the stage-1 stores to Uo below would
-        // otherwise hold each next load back (the compiler cannot tell Uo
-        // from Bin), one memory round trip per face
+        // The face fields rotate through three buffers, so that the field at
+        // the step's start stays where it is (Bold) and stage 1 copies nothing:
+        // its update wrote 24 B a cell more, 276 B in the FP32 split, 432 in FP64.
         double bup6[3], blo6[3];
         for (int d = 0; d < 3; ++d) {
             bup6[d] = a.Bin[d][c];
             blo6[d] = a.Bin[d][cl[d]];
         }
         for (int d = 0; d < 3; ++d) {
-            double bup = bup6[d];
-            double uoup;
-            if (STAGE == 1) {
-                uoup = bup;
-                a.Uo[5 + d][c] = bup;
-            } else {
-                uoup = a.Uo[5 + d][c];
-            }
+            const double bup = bup6[d], blo = blo6[d];
+            const double uoup = STAGE == 1 ? bup : a.Bold[d][c], uolo = STAGE == 1 ? blo : a.Bold[d][cl[d]];
             bn_up[d] = rk<STAGE>(uoup, bup, dt, Lup[d]);
-            double blo = blo6[d], uolo;
-            if (STAGE == 1) {
-                uolo = blo;
-                if (fidx[d] == 1) a.Uo[5 + d][cl[d]] = blo;
-            } else {
-                uolo = a.Uo[5 + d][cl[d]];
-            }
             const double llo = d < 2 ? Llo[d] : lB_z<G>(a, j, k, ey_mz, ey_mxmz, ex_mz, ex_mymz);
             bn_lo[d] = rk<STAGE>(uolo, blo, dt, llo);
             // the lowest face (index 0) keeps its stored value in prim
