@@ -772,7 +772,7 @@ int cumc3d_initial_update(cumc3d_ctx *x) {
         f32::initial_update(x);
     } else {
         hipLaunchKernelGGL(k_init_interior<double>, dim3(gi), dim3(256), 0, x->stream, make_args<double>(x));
-        hipLaunchKernelGGL(k_ghost<double>, dim3(nblk(ghost_count(*x))), dim3(256), 0, x->stream, make_args<double>(x));
+        launch_ghost<double>(x, make_args<double>(x));
     }
     x->nstep_total = 0;
     x->grav_error = 0;
@@ -823,6 +823,7 @@ int cumc3d_rk3_step(cumc3d_ctx *x, double dt) {
     hipLaunchKernelGGL(k_set_dt, dim3(1), dim3(1), 0, x->stream, x->S, dt, (int)x->dt_taken);
     x->dt_taken = false;
     x->cur_step = x->nstep_total;
+    x->whole = true;
     for (int s = 1; s <= 3; ++s)
         if (int rc = run_stage(x, s, s == 3 ? x->pub : nullptr)) return rc;
     x->nstep_total += 1;
@@ -846,6 +847,7 @@ int cumc3d_stage(cumc3d_ctx *x, int stage, double dt) {
         x->cur_step = x->nstep_total;
         x->dt_pending = false;
     }
+    x->whole = false;
     if (int rc = run_stage(x, stage, stage == 3 ? x->pub : nullptr)) return rc;
     x->next_stage = stage % 3 + 1;
     if (stage == 3) {
@@ -911,6 +913,7 @@ static int run_loop(cumc3d_ctx *x, int max_steps, double total_time, int sync_ea
     }
     int n = 0, grc = 0;
     double tcur = *t;
+    x->whole = true;
     for (; n < max_steps && !grc; ++n) {
         if (sync_each_step && !(tcur < total_time)) break;
         // FINDDT: the previous stage 3 already reduced the minimum

@@ -30,6 +30,7 @@ struct cumc3d_ctx {
     double *B[3][3], *Uo[5], *U[5], *floors[3];
     int cur = 0;                  // B[cur] holds the current face field,
     int old = 0;                  // B[old] that of the step's start
+    bool whole = false;           // the stages of a step run without the caller between them
     long march_threads = 0;         // y/z sweeps' thread count from CUMC3D_MARCH_THREADS (0: segments())
     int march[2] = {1, 1};          // segments per column of the y and z sweeps
     // learned reconstruction selector
@@ -416,20 +417,26 @@ static inline void tmark(cumc3d_ctx *x, int slot) {
 // SPATIAL up to l_operator: the three sweeps (fluxes, face and cell EMFs)
 // and the edge EMFs of the current state; `marks` records the stage's
 // timing events
+template <class W> static void launch_ghost(cumc3d_ctx *x, const ArgsT<W> &g, bool lean = false) {
+    const dim3 grid(nblk(ghost_count(*x)));
+    if (lean) hipLaunchKernelGGL((k_ghost<W, true>), grid, dim3(256), 0, x->stream, g);
+    else hipLaunchKernelGGL((k_ghost<W, false>), grid, dim3(256), 0, x->stream, g);
+}
+
 // The FP32 split's state kernels (update, ghost fill) live in their own
 // translation unit, whose double arithmetic keeps IEEE division.
 namespace f32 {
 void update(cumc3d_ctx *x, const ArgsT<float> &a, int stage, dim3 grid);
-void ghost(cumc3d_ctx *x, const ArgsT<float> &g);
+void ghost(cumc3d_ctx *x, const ArgsT<float> &g, bool lean);
 }  // namespace f32
 
 template <class W> static void stage_update(cumc3d_ctx *x, const ArgsT<W> &a, int stage, dim3 grid) {
     if constexpr (sizeof(W) == 4) f32::update(x, a, stage, grid);
     else launch_update<W>(x->d.coordinate_flag, stage, grid, x->stream, a);
 }
-template <class W> static void stage_ghost(cumc3d_ctx *x, const ArgsT<W> &g) {
-    if constexpr (sizeof(W) == 4) f32::ghost(x, g);
-    else hipLaunchKernelGGL(k_ghost<W>, dim3(nblk(ghost_count(*x))), dim3(256), 0, x->stream, g);
+template <class W> static void stage_ghost(cumc3d_ctx *x, const ArgsT<W> &g, bool lean) {
+    if constexpr (sizeof(W) == 4) f32::ghost(x, g, lean);
+    else launch_ghost<W>(x, g, lean);
 }
 
 template <class W> static void sweeps_t(cumc3d_ctx *x, const ArgsT<W> &a, hipStream_t st, bool marks) {
@@ -477,7 +484,7 @@ template <class W> static void run_stage_t(cumc3d_ctx *x, int stage, HostScalars
     ArgsT<W> g = make_args<W>(x);
     for (int d = 0; d < 3; ++d) g.Bout[d] = x->B[in][d];   // an inactive step's state
     g.pub = pub;
-    stage_ghost<W>(x, g);
+    stage_ghost<W>(x, g, x->whole && stage < 3 && x->d.n_dim < 3 && x->d.model != CUMC3D_MODEL_COLLAPSAR);
     tmark(x, 6);
     if (x->timing && x->tstage < TSTAGES) x->tstage += 1;
 }

@@ -14,8 +14,8 @@ void update(cumc3d_ctx *x, const ArgsT<float> &a, int stage, dim3 grid) {
     launch_update<float>(x->d.coordinate_flag, stage, grid, x->stream, a);
 }
 
-void ghost(cumc3d_ctx *x, const ArgsT<float> &g) {
-    hipLaunchKernelGGL(k_ghost<float>, dim3(nblk(ghost_count(*x))), dim3(256), 0, x->stream, g);
+void ghost(cumc3d_ctx *x, const ArgsT<float> &g, bool lean) {
+    launch_ghost<float>(x, g, lean);
 }
 
 void finddt(cumc3d_ctx *x) {
@@ -31,7 +31,7 @@ void split_prim(cumc3d_ctx *x, const double *aos, const double *eps64) {
 void initial_update(cumc3d_ctx *x) {
     const unsigned gi = nblk((long)x->nx * x->ny * x->nz);
     hipLaunchKernelGGL(k_init_interior<float>, dim3(gi), dim3(256), 0, x->stream, make_args<float>(x));
-    hipLaunchKernelGGL(k_ghost<float>, dim3(nblk(ghost_count(*x))), dim3(256), 0, x->stream, make_args<float>(x));
+    launch_ghost<float>(x, make_args<float>(x));
 }
 
 void join_prim(cumc3d_ctx *x, double *tmp) {
