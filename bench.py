@@ -86,11 +86,8 @@ def kernel_model_bytes(cfg, name: str, w: int) -> float:
         faces = {"flux_x": (nx + 1) * ny * nz, "flux_y": nx * (ny + 1) * nz, "flux_z": nx * ny * (nz + 1)}[name]
         return 7 * w * cells + (8 + 7 * w) * faces
     if name == "edge":
-        # edge: 6 face-EMF arrays + 3 cell-EMF arrays -> 3 edge EMFs on
-        # (n+1)^3, plus the face-EMF fill of the (n+2)^3 box's shell (the
-        # mapped interior face EMF read, the ghost one written: 4 per cell)
-        shell = (nx + 2) * (ny + 2) * (nz + 2) - n
-        return 12 * w * (nx + 1) * (ny + 1) * (nz + 1) + 4 * w * shell
+        # 6 face-EMF arrays + 3 cell-EMF arrays -> 3 edge EMFs on (n+1)^3
+        return 12 * w * (nx + 1) * (ny + 1) * (nz + 1)
     if name == "update":
         # stage 2/3 of the fused update
         if split:
@@ -120,6 +117,11 @@ def traffic_summary(workload: str, n: int) -> str:
     return os.path.join(ROOT, "profiles", f"traffic_{workload}{n}_hlld.md")
 
 
+def sweep_axis(name: str) -> str:
+    """flux_y or flux_z: the fourth template argument of k_flux_yz<T, R, S, D, FLAT>."""
+    return "flux_y" if name.split(",")[3].strip().startswith("1") else "flux_z"
+
+
 def measured_traffic(kernel: str, w: int, workload: str, n: int):
     """HBM bytes per launch of a kernel class from the committed rocprofv3
     FETCH_SIZE/WRITE_SIZE summary of this workload (calibrated against a copy
@@ -136,7 +138,7 @@ def measured_traffic(kernel: str, w: int, workload: str, n: int):
         cols = [c.strip().strip("`") for c in line.strip().strip("|").split("|")]
         if len(cols) < 6 or not cols[0].startswith(prefix) or typ not in cols[0]:
             continue
-        if kernel in ("flux_y", "flux_z") and not cols[0].rstrip(">").endswith("1" if kernel == "flux_y" else "2"):
+        if kernel in ("flux_y", "flux_z") and sweep_axis(cols[0]) != kernel:
             continue
         try:
             vals.append(float(cols[5]) * 1e6)
@@ -569,7 +571,7 @@ def trace_summary(path: str, n: int, workload: str = "turbulence") -> str:
         if "k_flux_x<" in name:
             kb = kernel_model_bytes(cfg, "flux_x", w)
         elif "k_flux_yz<" in name:
-            kb = kernel_model_bytes(cfg, "flux_y" if name.rstrip(")").split(",")[3].strip().startswith("1") else "flux_z", w)
+            kb = kernel_model_bytes(cfg, sweep_axis(name), w)
         elif "k_update<" in name:
             kb = kernel_model_bytes(cfg, "update", w)
             stage = int(name.split("k_update<")[1].split(",")[0])
@@ -656,7 +658,7 @@ def pmc_summary(paths, n: int, workload: str = "turbulence") -> str:
         if "k_flux_x<" in name:
             kb = kernel_model_bytes(cfg, "flux_x", w)
         elif "k_flux_yz<" in name:
-            kb = kernel_model_bytes(cfg, "flux_y" if name.split("(")[0].rstrip(">").endswith("1") else "flux_z", w)
+            kb = kernel_model_bytes(cfg, sweep_axis(name), w)
         elif "k_update<" in name:
             kb = kernel_model_bytes(cfg, "update", w)
             stg = int(name.split("k_update<")[1].split(",")[0])

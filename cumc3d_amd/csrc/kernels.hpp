@@ -629,9 +629,10 @@ __device__ __forceinline__ void ppm_next(const ArgsT<T> &a, long c, int i, long 
 // What bounds it: VALU issue, given waves to issue from.  With the kept face
 // in registers the FP64 march needed 168 to 256 VGPRs and up to 78 AGPRs (one
 // or two waves per SIMD); in LDS it fits three.  Measured at 256^3, y / z sweep,
-// HLLD + WENO-Z: 2.05 / 1.95 -> 1.56 / 1.56 ms.  In single precision the face
-// stays in registers for the fixed schemes: from LDS, TVD-MC took 0.360 against
-// 0.353 ms and PPM 0.495 against 0.474 ms (the selector 0.400 against 0.467).
+// HLLD + WENO-Z: 2.05 / 1.95 -> 1.56 / 1.56 ms (1.38 / 1.41 with fewer
+// operations per face since).  In single precision the face stays in registers
+// for the fixed schemes: from LDS, TVD-MC took 0.360 against 0.353 ms and PPM,
+// before it shared edges, 0.495 against 0.474 (the selector 0.400 against 0.467).
 // FLAT (the selector, where the planes are no whole number of waves): the
 // segments too are laid end to end over the threads.  A wave reconstructs all
 // its cells by its highest class, so which cells share a wave is part of the
